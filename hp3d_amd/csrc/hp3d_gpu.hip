@@ -1,12 +1,11 @@
 // hp3d_gpu.hip -- MI355X (gfx950) element computation for hp3D hexahedra.
 //
 // Kernels
-//   elem_kernel   one workgroup per (element, 128x128 block of K): 1D factor
-//                 tables and per-point geometry in LDS, A = B^T(geometry)
-//                 streamed through LDS in chunks of quadrature points, and
-//                 K += A A^T on MFMA (v_mfma_f64_16x16x4f64 or
-//                 v_mfma_f32_16x16x4f32), upper-triangle tiles only, written
-//                 out in both triangles with coalesced column segments.
+//   sf_elem_kernel  (hp3d_sumfac.h) element matrices by sum factorisation over
+//                 the three directions, any N, FP64 arithmetic.
+//   elem_kernel   the BF16 trial for N > 128: one workgroup per (element, 128 x
+//                 128 block of K), A = B^T(geometry) streamed through LDS in
+//                 chunks of quadrature points, K += A A^T on bf16 MFMA.
 //   elem_single_kernel  one workgroup per element with N <= 128: K kept in
 //                 registers over the quadrature, then (nb <= 32) the bubble
 //                 block condensed in the same launch.
@@ -666,6 +665,8 @@ __device__ inline s4_t bf4(const float *col, int ld, int off)
     return s4_t{f2bf(col[off]), f2bf(col[ld + off]), f2bf(col[2 * ld + off]), f2bf(col[3 * ld + off])};
 }
 
+#include "hp3d_sumfac.h"
+
 // Geometry pass of the block-tiled path: every quadrature point of an
 // element once (geom3D.F90:77-91, geom.F90:57-113, elem_opt.F90:101-122),
 // into the element's slab of the workspace, which all of the element's K
@@ -698,36 +699,29 @@ __global__ __launch_bounds__(WG) void geometry_kernel(ElemArgs a)
     if (tid == 0) gp[(size_t)MAXQ * GS] = es.negjac ? 1.0 : 0.0;
 }
 
-// General element kernel: one workgroup of 8 waves per (element, 128 x 128
-// block of K).  An off-diagonal block's 64 tiles of 16 x 16 are 8 per wave
-// (wave w: tile row w); a diagonal block's 36 upper tiles are 5 or 4 per wave
-// (waves p and p + 4 share tile rows p and 7 - p, 9 tiles).  With 8 tiles a
-// wave fits in 128 VGPRs, so two workgroups give 4 waves per SIMD.
-// The geometry comes from the element's slab (geometry_kernel).
-// Each row of the block's A is built by 2 (off-diagonal) or 4 (diagonal)
-// threads, each for its share of the chunk's points, with the row's
-// descriptor read once; the A chunks are double buffered (FP32 24, FP64 12
-// columns per chunk), so a chunk's build follows the MFMAs of the previous
-// one with one barrier between chunks.
-// BF (with T = float): the contraction's operands are rounded to bfloat16 and
-// multiplied on v_mfma_f32_16x16x16_bf16 with FP32 accumulation (the BF16
-// trial); the A chunk is padded from KC to 32 columns with zeros.
+// The BF16 trial's kernel for N > 128: one workgroup of 8 waves per (element,
+// 128 x 128 block of K), the contraction's operands rounded to bfloat16 and
+// multiplied on v_mfma_f32_16x16x16_bf16 with FP32 accumulation.  An
+// off-diagonal block's 64 tiles of 16 x 16 are 8 per wave (wave w: tile row
+// w); a diagonal block's 36 upper tiles are 5 or 4 per wave (waves p and p + 4
+// share tile rows p and 7 - p, 9 tiles).  The geometry comes from the
+// element's slab (geometry_kernel).  Each row of the block's A is built by 2
+// (off-diagonal) or 4 (diagonal) threads, each for its share of the chunk's
+// points, with the row's descriptor read once; the A chunk is padded from KC
+// to 32 columns with zeros.
 constexpr int WGE = 512; // threads per workgroup of the block-tiled kernel
-template <typename T, int SPACE, bool BF = false>
+template <int SPACE>
 __global__ __launch_bounds__(WGE, 4) void elem_kernel(ElemArgs a)
 {
+    typedef float T;
     typedef Mfma<T> M;
     typedef typename M::acc_t acc_t;
     constexpr int NC = SPACE == 0 ? 3 : 6;             // A columns per point
-    constexpr int KCE = (BF || sizeof(T) == 4) ? KC : KC / 2; // A columns per chunk
-    constexpr int NBUF = BF ? 1 : 2;                   // A buffers
-    constexpr int QC = KCE / NC;                       // points per A chunk
+    constexpr int QC = KC / NC;                        // points per A chunk
     constexpr int GQ = 64;                             // points per geometry pass
     constexpr int GS = geo_stride(SPACE);              // geometry doubles per point
-    constexpr int KCA = BF ? 32 : KCE;                 // allocated A columns
-    constexpr int BUFE = KCA * LDA;                    // one A buffer, in T
+    constexpr int KCA = 32;                            // allocated A columns
     constexpr int NS = 8;                              // tile slots per wave
-    static_assert(!BF || sizeof(T) == 4, "bfloat16 operands come from an FP32 chunk");
     static_assert(GQ % QC == 0 && QC % 2 == 0, "a geometry pass holds whole chunks");
 
     __shared__ ElemShared es;
@@ -736,7 +730,7 @@ __global__ __launch_bounds__(WGE, 4) void elem_kernel(ElemArgs a)
     __shared__ unsigned pix[MAXQ];     // packed 1D point indices
     __shared__ double geo[GQ * GS];
     __shared__ double bv[3][BR];       // partial load sums of a diagonal block's rows
-    __shared__ T ac[NBUF * BUFE];
+    __shared__ T ac[KCA * LDA];
 
     const int e = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -769,8 +763,7 @@ __global__ __launch_bounds__(WGE, 4) void elem_kernel(ElemArgs a)
         Pt p = point_ix(l, es.nq);
         pix[l] = (unsigned)p.l1 | ((unsigned)p.l2 << 4) | ((unsigned)p.l3 << 8);
     }
-    if (BF)
-        for (int i = tid; i < (KCA - KC) * LDA; i += WGE) ac[KC * LDA + i] = (T)0;
+    for (int i = tid; i < (KCA - KC) * LDA; i += WGE) ac[KC * LDA + i] = (T)0;
     __syncthreads();
 
     const double *gsrc = a.gws + (size_t)e * geo_slab(SPACE);
@@ -812,14 +805,9 @@ __global__ __launch_bounds__(WGE, 4) void elem_kernel(ElemArgs a)
         valid |= (v ? 1u : 0u) << s;
     }
     const unsigned vmask = valid;
-    typedef Carry<std::conditional_t<BF, double, T>, acc_t> CY; // no carry under bfloat16 rounding
     acc_t acc[NS];
-    typename CY::hi_t hi[NS];
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        acc[s] = acc_t{0, 0, 0, 0};
-        CY::zero(hi[s]);
-    }
+    for (int s = 0; s < NS; ++s) acc[s] = acc_t{0, 0, 0, 0};
     const bool do_load = diag && a.bout != nullptr;
 
     // this thread's row of A (row r of the block's row set: I rows, then J
@@ -855,31 +843,19 @@ __global__ __launch_bounds__(WGE, 4) void elem_kernel(ElemArgs a)
         else build_pts(std::integral_constant<int, WGE / (2 * BR)>{}, g0, l0, gend, buf);
     };
     auto mfma = [&](const T *buf) {
-        if constexpr (BF) {
 #pragma unroll
-            for (int k0 = 0; k0 < KCA; k0 += 16) {
-                const float *col = (const float *)buf + (k0 + 4 * (lane >> 4)) * LDA + l15;
-                s4_t aA = bf4(col, LDA, tiA * 16);
-                s4_t aB = bf4(col, LDA, tiB * 16);
+        for (int k0 = 0; k0 < KCA; k0 += 16) {
+            const float *col = buf + (k0 + 4 * (lane >> 4)) * LDA + l15;
+            s4_t aA = bf4(col, LDA, tiA * 16);
+            s4_t aB = bf4(col, LDA, tiB * 16);
 #pragma unroll
-                for (int s = 0; s < NS; ++s)
-                    if (vmask & (1u << s))
-                        acc[s] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(s < nA ? aA : aB, bf4(col, LDA, offS[s]),
-                                                                          acc[s], 0, 0, 0);
-            }
-        } else {
-#pragma unroll
-            for (int k0 = 0; k0 < KCE; k0 += 4) {
-                const T *col = buf + (k0 + (lane >> 4)) * LDA + l15;
-                const T aA = col[tiA * 16], aB = col[tiB * 16];
-#pragma unroll
-                for (int s = 0; s < NS; ++s)
-                    if (vmask & (1u << s)) acc[s] = M::mma(s < nA ? aA : aB, col[offS[s]], acc[s]);
-            }
+            for (int s = 0; s < NS; ++s)
+                if (vmask & (1u << s))
+                    acc[s] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(s < nA ? aA : aB, bf4(col, LDA, offS[s]),
+                                                                      acc[s], 0, 0, 0);
         }
     };
 
-    int nfold = 0;
     for (int g0 = 0; g0 < nint; g0 += GQ) {
         const int gend = min(GQ, nint - g0);
         for (int i = tid; i < gend * GS; i += WGE) geo[i] = gsrc[(size_t)g0 * GS + i];
@@ -888,29 +864,11 @@ __global__ __launch_bounds__(WGE, 4) void elem_kernel(ElemArgs a)
         build(g0, 0, gend, ac);
         __syncthreads();
         for (int c = 0; c < nch; ++c) {
-            if constexpr (NBUF == 2) {
-                // waves w and w + 4 share a SIMD: one issues its MFMAs while the
-                // other builds the next chunk, then they swap
-                T *cur = ac + (c & 1) * BUFE, *nxt = ac + ((c + 1) & 1) * BUFE;
-                const bool first = wv >= 4 && c + 1 < nch, second = wv < 4 && c + 1 < nch;
-                if (first) build(g0, (c + 1) * QC, gend, nxt);
-                __asm__ volatile("" ::: "memory");
-                mfma(cur);
-                __asm__ volatile("" ::: "memory");
-                if (second) build(g0, (c + 1) * QC, gend, nxt);
-            } else {
-                mfma(ac);
-            }
-            if ((++nfold & 3) == 0) { // FP32: every 4 chunks of 24 columns
-#pragma unroll
-                for (int s = 0; s < NS; ++s) CY::fold(hi[s], acc[s]);
-            }
+            mfma(ac);
             __syncthreads();
-            if constexpr (NBUF == 1) {
-                if (c + 1 < nch) {
-                    build(g0, (c + 1) * QC, gend, ac);
-                    __syncthreads();
-                }
+            if (c + 1 < nch) {
+                build(g0, (c + 1) * QC, gend, ac);
+                __syncthreads();
             }
         }
     }
@@ -929,7 +887,7 @@ __global__ __launch_bounds__(WGE, 4) void elem_kernel(ElemArgs a)
     for (int s = 0; s < NS; ++s) {
         if (!(valid & (1u << s))) continue;
         const int ti = s < nA ? tiA : tiB, tj = s < nA ? tjA + s : tjB + (s - nA);
-        write_sym_tile<acc_t, T, M>(CY::sum(hi[s], acc[s]), I * BR + ti * 16, J * BR + tj * 16, n, kout, ld,
+        write_sym_tile<acc_t, T, M>(acc[s], I * BR + ti * 16, J * BR + tj * 16, n, kout, ld,
                                     stage, lane);
     }
 }
@@ -2717,6 +2675,20 @@ static int launch_single(int space, int precision, const ElemArgs &args, const C
     return launch_single_r<BR>(space, precision, args, cd, st);
 }
 
+// the sum-factorised element kernel; few elements are split over several
+// workgroups each (their column chunks) until the chip's 256 CUs have three
+template <typename T>
+static int launch_sf(int space, const ElemArgs &args, int max_ndof, hipStream_t st)
+{
+    const int most = space == HP3D_H1 ? SF_I : 3 * SF_I;
+    const int parts = std::max(1, std::min(most, 768 / std::max(args.nel, 1)));
+    const dim3 grid(args.nel, parts);
+    if (space == HP3D_H1) hipLaunchKernelGGL((sf_elem_kernel<T, 0, 256, 5540, 3>), grid, dim3(256), 0, st, args);
+    else hipLaunchKernelGGL((sf_elem_kernel<T, 1, 384, 8674, 3>), grid, dim3(384), 0, st, args);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
 static int launch_elem(int space, int precision, const ElemArgs &args, int max_ndof,
                        hipStream_t st)
 {
@@ -2724,18 +2696,17 @@ static int launch_elem(int space, int precision, const ElemArgs &args, int max_n
         CondArgs cd{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
         return launch_single(space, precision, args, cd, max_ndof, 0, st);
     }
-    if (!args.gws) return HP3D_E_ARG; // the block-tiled path needs the geometry workspace
-    if (space == HP3D_H1) hipLaunchKernelGGL((geometry_kernel<0>), dim3(args.nel), dim3(WG), 0, st, args);
-    else hipLaunchKernelGGL((geometry_kernel<1>), dim3(args.nel), dim3(WG), 0, st, args);
+    if (precision == HP3D_FP64) return launch_sf<double>(space, args, max_ndof, st);
+    if (precision == HP3D_FP32) return launch_sf<float>(space, args, max_ndof, st);
+    // the BF16 trial: geometry pass, then the block-tiled MFMA kernel
+    if (!args.gws) return HP3D_E_ARG;
     dim3 grid(args.nel, nblocks_for(max_ndof)), block(WGE);
     if (space == HP3D_H1) {
-        if (precision == HP3D_FP64) hipLaunchKernelGGL((elem_kernel<double, 0>), grid, block, 0, st, args);
-        else if (precision == HP3D_BF16) hipLaunchKernelGGL((elem_kernel<float, 0, true>), grid, block, 0, st, args);
-        else hipLaunchKernelGGL((elem_kernel<float, 0>), grid, block, 0, st, args);
+        hipLaunchKernelGGL((geometry_kernel<0>), dim3(args.nel), dim3(WG), 0, st, args);
+        hipLaunchKernelGGL((elem_kernel<0>), grid, block, 0, st, args);
     } else {
-        if (precision == HP3D_FP64) hipLaunchKernelGGL((elem_kernel<double, 1>), grid, block, 0, st, args);
-        else if (precision == HP3D_BF16) hipLaunchKernelGGL((elem_kernel<float, 1, true>), grid, block, 0, st, args);
-        else hipLaunchKernelGGL((elem_kernel<float, 1>), grid, block, 0, st, args);
+        hipLaunchKernelGGL((geometry_kernel<1>), dim3(args.nel), dim3(WG), 0, st, args);
+        hipLaunchKernelGGL((elem_kernel<1>), grid, block, 0, st, args);
     }
     HIPCHK(hipGetLastError());
     return 0;

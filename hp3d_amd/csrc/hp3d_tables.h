@@ -436,4 +436,130 @@ HP3D_HD inline unsigned desc_h1_scan(int k, const ElemOrders &o)
     return put(ps ? ax1 : ax0, t_phi(kl - j0 * h1 + 2, rs), pt ? ax1 : ax0, t_phi(j0 + 2, rt), dn, fa);
 }
 
+// ---- the dof layout from the tensor side (sum-factorised kernels)
+//
+// Every dof is +- a product of 1D functions of one index per direction:
+// chi_0 = 1 - x, chi_1 = x, chi_i = phi_i (i = 2..MAXP) in H1.  The reversed
+// factors of the orientation codes are the same functions up to a sign,
+// phi_i(1 - x) = (-1)^i phi_i(x) and P_i(1 - x) = (-1)^i P_i(x), and the
+// Legendre factor of an H(curl) dof is a derivative of this family:
+// P_{i-1} = d chi_i / dx, i >= 1.  So an H(curl) dof of component a is
+// d(chi_i0 chi_i1 chi_i2)/dx_a with i_a >= 1.
+
+// first dof of every entity: 12 edges, 6 faces, the interior
+struct DofBases {
+    short edge[12], face[6], interior;
+};
+
+HP3D_HD inline void dof_bases(int space, const ElemOrders &o, DofBases &b)
+{
+    int at = space == 0 ? 8 : 0;
+    for (int e = 0; e < 12; ++e) {
+        b.edge[e] = (short)at;
+        at += space == 0 ? o.pe[e] - 1 : o.pe[e];
+    }
+    for (int f = 0; f < 6; ++f) {
+        const int h = o.fh[f], v = o.fv[f];
+        b.face[f] = (short)at;
+        at += space == 0 ? (h - 1) * (v - 1) : h * (v - 1) + (h - 1) * v;
+    }
+    b.interior = (short)at;
+}
+
+// edge with direction d at the affine indexes (i, j) of the two other
+// directions (ascending), and face with normal d at affine index i
+HP3D_HD constexpr int edge_at(int d, int i, int j)
+{
+    return d == 0 ? (j == 0 ? (i == 0 ? 0 : 2) : (i == 0 ? 4 : 6))
+         : d == 1 ? (j == 0 ? (i == 0 ? 3 : 1) : (i == 0 ? 7 : 5))
+                  : (i == 0 ? (j == 0 ? 8 : 11) : (j == 0 ? 9 : 10));
+}
+HP3D_HD constexpr int face_at(int d, int i)
+{
+    return d == 2 ? i : d == 1 ? (i == 0 ? 2 : 4) : (i == 0 ? 5 : 3);
+}
+
+constexpr int ROW_NEG = 1 << 14; // sign bit of dof_row
+
+// the dof with 1D indexes (i0, i1, i2) (0..MAXP each) and, in H(curl),
+// component a (i_a >= 1): its number, plus ROW_NEG when the dof is minus the
+// product, or -1 when the element has no such dof
+HP3D_HD inline int dof_row(int space, int a, int i0, int i1, int i2, const ElemOrders &o, const DofBases &b)
+{
+    const int ix[3] = {i0, i1, i2};
+    if (space == 0) a = -1;
+    else if (ix[a] < 1) return -1;
+    // directions in which the dof is not one of the two affine functions
+    const bool in0 = a == 0 || i0 >= 2, in1 = a == 1 || i1 >= 2, in2 = a == 2 || i2 >= 2;
+    const int inner = (int)in0 + (int)in1 + (int)in2;
+    if (inner == 0) { // vertex: (00), (10), (11), (01) of the bottom, then the top
+        return (i1 ? (i0 ? 2 : 3) : i0) + 4 * i2;
+    }
+    if (inner == 1) {
+        const int d = in0 ? 0 : in1 ? 1 : 2;
+        const int e = edge_at(d, d == 0 ? i1 : i0, d == 2 ? i1 : i2);
+        const int k = d == 0 ? i0 : d == 1 ? i1 : i2;
+        if (k > o.pe[e]) return -1;
+        // H1: phi_k, k = 2..p; H(curl): P_{k-1}, k = 1..p, and the sign of the
+        // reversed tangent
+        if (space == 0) return b.edge[e] + k - 2 + ((o.oe[e] && (k & 1)) ? ROW_NEG : 0);
+        return b.edge[e] + k - 1 + ((o.oe[e] && (k & 1)) ? ROW_NEG : 0);
+    }
+    if (inner == 2) {
+        const int d = !in0 ? 0 : !in1 ? 1 : 2;
+        const int f = face_at(d, d == 0 ? i0 : d == 1 ? i1 : i2);
+        const int ax0 = d == 0 ? 1 : 0, ax1 = d == 2 ? 1 : 2;
+        const FaceOri fo = face_ori(o.of[f]);
+        const int ds = fo.ps ? ax1 : ax0, dt = fo.pt ? ax1 : ax0;
+        const int i = ds == 0 ? i0 : ds == 1 ? i1 : i2, j = dt == 0 ? i0 : dt == 1 ? i1 : i2;
+        const int h = o.fh[f], v = o.fv[f];
+        if (i > h || j > v) return -1;
+        // a reversed axis gives (-1)^index: for phi from the function, for
+        // the Legendre factor P_{i-1} from (-1)^{i-1} and the sign of the
+        // reversed tangent
+        const int neg = ((fo.rs && (i & 1)) != (fo.rt && (j & 1))) ? ROW_NEG : 0;
+        if (space == 0) return b.face[f] + (i - 2) + (h - 1) * (j - 2) + neg;
+        if (a == ds) return b.face[f] + (i - 1) + h * (j - 2) + neg;
+        return b.face[f] + h * (v - 1) + (i - 2) + (h - 1) * (j - 1) + neg;
+    }
+    if (i0 > o.b[0] || i1 > o.b[1] || i2 > o.b[2]) return -1;
+    const int bx = o.b[0], by = o.b[1], bz = o.b[2];
+    if (space == 0) return b.interior + (i0 - 2) + (bx - 1) * ((i1 - 2) + (by - 1) * (i2 - 2));
+    // the families of the three components, one after the other
+    const int n0 = bx * (by - 1) * (bz - 1), n1 = (bx - 1) * by * (bz - 1);
+    const int c0 = a == 0 ? bx : bx - 1, c1 = a == 1 ? by : by - 1;
+    const int g0 = a == 0 ? i0 - 1 : i0 - 2, g1 = a == 1 ? i1 - 1 : i1 - 2, g2 = a == 2 ? i2 - 1 : i2 - 2;
+    return b.interior + (a == 0 ? 0 : a == 1 ? n0 : n0 + n1) + g0 + c0 * (g1 + c1 * g2);
+}
+
+// 1D tables of the sum-factorised kernels at the n Gauss points of a
+// direction: f[n][0][i][q] = chi_i(x_q), f[n][1][i][q] = chi_i'(x_q), and the
+// weights of the rule on [0, 1]
+struct SfTables {
+    double f[MAXP + 2][2][MAXP + 1][8];
+    double w[MAXP + 2][8];
+};
+constexpr SfTables make_sf_tables()
+{
+    constexpr double gx[10][10] = HP3D_GAUSS_X, gw[10][10] = HP3D_GAUSS_W;
+    SfTables t{};
+    for (int n = 1; n <= MAXP + 1; ++n)
+        for (int q = 0; q < n; ++q) {
+            const double x = 0.5 * (1.0 + gx[n - 1][q]), y = 2.0 * x - 1.0;
+            double p[MAXP + 1] = {1.0, y};
+            for (int i = 2; i <= MAXP; ++i)
+                p[i] = ((double)(2 * i - 1) * y * p[i - 1] - (double)(i - 1) * p[i - 2]) / (double)i;
+            t.f[n][0][0][q] = 1.0 - x;
+            t.f[n][1][0][q] = -1.0;
+            t.f[n][0][1][q] = x;
+            t.f[n][1][1][q] = 1.0;
+            for (int i = 2; i <= MAXP; ++i) {
+                t.f[n][0][i][q] = (p[i] - p[i - 2]) / (double)(4 * i - 2);
+                t.f[n][1][i][q] = p[i - 1];
+            }
+            t.w[n][q] = 0.5 * gw[n - 1][q];
+        }
+    return t;
+}
+
 } // namespace hp3d

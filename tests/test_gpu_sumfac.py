@@ -1,0 +1,72 @@
+"""The sum-factorised element matrices against the oracle, at the sizes and
+codes where the kernel's splits change: every pair of pencil lengths and column
+chunks (anisotropic orders), orders of edges and faces above the interior's,
+isoparametric maps, a leading dimension above N and split elements (a few
+elements run several workgroups each).
+
+Tolerance: the reference sums O(10^3) products of magnitude |K|_F at most per
+entry in FP64, as the kernel does in another order, so both stay within about
+sqrt(10^3) eps of the exact value: 1e-13 of |K|_F covers both with room.  FP32
+K is the FP64 value rounded once: 2^-24 relative to the largest entry, held
+to 1e-7."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+from hp3d_amd import mesh
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+def random_codes(rng, nel, pmax):
+    no = np.zeros((nel, 19), np.int32)
+    no[:, :12] = rng.integers(1, pmax + 1, (nel, 12))
+    no[:, 12:18] = 10 * rng.integers(1, pmax + 1, (nel, 6)) + rng.integers(1, pmax + 1, (nel, 6))
+    b = rng.integers(1, pmax + 1, (nel, 3))
+    no[:, 18] = 100 * b[:, 0] + 10 * b[:, 1] + b[:, 2]
+    return no, rng.integers(0, 2, (nel, 12)).astype(np.int32), rng.integers(0, 8, (nel, 6)).astype(np.int32)
+
+
+def check(space, no, oe, of, xnod, coef, precision=0):
+    import torch
+
+    import hp3d_amd
+
+    load = oracle.LOAD_SINSINSIN if space == 0 else oracle.LOAD_CURL_SIN
+    batch = hp3d_amd.ElementBatch(space, no, oe, of, xnod, coef, load=load, rules=({"path": "two_pass"},))
+    out = batch.alloc_outputs(precision, want_stc=False)
+    batch.element_matrices(out, precision)
+    torch.cuda.synchronize()
+    assert (batch.check_status() == 0).all()
+    ref = oracle.element_loop(space, no, oe, of, xnod, coef, load, ldk=int(batch.n.max()), want_stc=False)
+    for e in range(batch.nel):
+        n = int(batch.n[e])
+        k = batch.k_of(out, e)
+        assert rel(k, ref["k"][e].T[:n, :n]) < (1e-13 if precision == 0 else 1e-7), (e, n)
+        assert np.array_equal(k, k.T), e
+        b = ref["b"][e][:n]
+        assert np.linalg.norm(batch.vec_of(out, "b", e) - b) <= 1e-13 * max(np.linalg.norm(b), 1e-3)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("space", [0, 1])
+def test_any_codes(gpu, space, precision):
+    rng = np.random.default_rng(50 + space)
+    nel = 24
+    no, oe, of = random_codes(rng, nel, 6)
+    v = mesh.VERT_XYZ[None] + 0.15 * rng.uniform(-1, 1, (nel, 8, 3))
+    check(space, no, oe, of, v, rng.uniform(0.5, 2.0, nel), precision)
+
+
+@pytest.mark.parametrize("space", [0, 1])
+@pytest.mark.parametrize("porder", [(6, 6, 6), (6, 5, 1), (1, 6, 6), (5, 1, 6), (2, 6, 4), (6, 3, 3), (4, 5, 2), (5, 5, 5)])
+def test_anisotropic(gpu, space, porder):
+    m = mesh.structured((2, 1, 1), porder=porder, perturb=0.0, perm_seed=3 + sum(porder), coef=[0.7, 1.9])
+    x = m.xnod() + 0.05 * np.random.default_rng(sum(porder)).uniform(-1, 1, (2, 8, 3))
+    check(space, m.norder, m.nori_e, m.nori_f, x, m.coef)
