@@ -665,6 +665,12 @@ __device__ inline s4_t bf4(const float *col, int ld, int off)
     return s4_t{f2bf(col[off]), f2bf(col[ld + off]), f2bf(col[2 * ld + off]), f2bf(col[3 * ld + off])};
 }
 
+constexpr int NBF = 32;      // largest bubble block condensed in the fused path
+struct CondArgs {
+    const long long *off_c, *off_s;
+    double *aii, *bi, *aschur, *bschur;
+};
+
 #include "hp3d_sumfac.h"
 
 // Geometry pass of the block-tiled path: every quadrature point of an
@@ -903,12 +909,6 @@ __global__ __launch_bounds__(WGE, 4) void elem_kernel(ElemArgs a)
 //   X = L_u^-T D^-1/2 S = Abb^-1 [Abi | Bb] = [ASchur | BSchur].
 // The A chunks are double buffered: the MFMAs of chunk c are issued before
 // the VALU/LDS work that builds chunk c+1, so the two overlap.
-constexpr int NBF = 32;      // largest bubble block condensed in the fused path
-struct CondArgs {
-    const long long *off_c, *off_s;
-    double *aii, *bi, *aschur, *bschur;
-};
-
 template <typename T> struct SingleCfg {
     static constexpr int KCS = sizeof(T) == 4 ? 48 : 24; // A columns per chunk
 };
@@ -1515,38 +1515,6 @@ template <typename T, int SPACE, int R, bool BF = false>
 __global__ __launch_bounds__(WG, R == BR ? 2 : 3) void elem_single_kernel(ElemArgs a, CondArgs cd)
 {
     single_element<T, SPACE, R, BF>(a, cd, blockIdx.x, threadIdx.x);
-}
-
-// arguments of the persistent form, as one kernel argument at offset 0
-struct SingleArgs {
-    ElemArgs a;
-    CondArgs cd;
-};
-typedef const __attribute__((address_space(4))) SingleArgs *kargs_t;
-
-// persistent form: a fixed grid (2 workgroups per CU) walks the elements with
-// a grid stride; the barrier after each element keeps the next element's
-// setup from overwriting LDS a slower wave still reads.  Per element the
-// arguments are read again from the kernel-argument segment (scalar loads)
-// and the thread index passes through an empty asm, so the compiler keeps
-// nothing derived from them live from one element to the next: the element
-// body needs every register.
-template <typename T, int SPACE, int R>
-__global__ __launch_bounds__(WG, R == BR ? 2 : 3) void elem_single_persistent(SingleArgs sa)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    const int nel = sa.a.nel, stride = gridDim.x;
-    for (int e = blockIdx.x; e < nel; e += stride) {
-        kargs_t kp = (kargs_t)__builtin_amdgcn_kernarg_segment_ptr();
-        __asm__ volatile("" : "+s"(kp));
-        const ElemArgs al = kp->a;
-        const CondArgs cl = kp->cd;
-        int tid = threadIdx.x;
-        __asm__ volatile("" : "+v"(tid));
-        single_element<T, SPACE, R>(al, cl, e, tid);
-        __syncthreads();
-    }
-#endif
 }
 
 // ------------------------------------------------------------ condensation
@@ -2629,50 +2597,69 @@ static int nblocks_for(int max_ndof)
     return t * (t + 1) / 2;
 }
 
+// the BF16 trial's single-block kernel
 template <int R>
-static int launch_single_r(int space, int precision, const ElemArgs &args, const CondArgs &cd,
-                           hipStream_t st)
+static int launch_single_bf16(int space, const ElemArgs &args, const CondArgs &cd, hipStream_t st)
 {
-    dim3 block(WG);
-    if (precision == HP3D_BF16) {
-        dim3 grid(args.nel);
-        if (space == HP3D_H1) hipLaunchKernelGGL((elem_single_kernel<float, 0, R, true>), grid, block, 0, st, args, cd);
-        else hipLaunchKernelGGL((elem_single_kernel<float, 1, R, true>), grid, block, 0, st, args, cd);
-    } else if (g_persistent) {
+    const dim3 grid(args.nel), block(WG);
+    if (space == HP3D_H1) hipLaunchKernelGGL((elem_single_kernel<float, 0, R, true>), grid, block, 0, st, args, cd);
+    else hipLaunchKernelGGL((elem_single_kernel<float, 1, R, true>), grid, block, 0, st, args, cd);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
+// one workgroup per element, or as many as the chip holds with the persistent
+// option (per_cu: workgroups that fit a CU's LDS)
+static int fused_grid(int nel, int per_cu, dim3 &grid)
+{
+    if (g_persistent) {
         int dev = 0, ncu = 0;
         HIPCHK(hipGetDevice(&dev));
         HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-        dim3 grid(std::min(args.nel, (R == BR ? 2 : 3) * std::max(ncu, 1)));
-        const SingleArgs sa{args, cd};
-        if (space == HP3D_H1) {
-            if (precision == HP3D_FP64) hipLaunchKernelGGL((elem_single_persistent<double, 0, R>), grid, block, 0, st, sa);
-            else hipLaunchKernelGGL((elem_single_persistent<float, 0, R>), grid, block, 0, st, sa);
-        } else {
-            if (precision == HP3D_FP64) hipLaunchKernelGGL((elem_single_persistent<double, 1, R>), grid, block, 0, st, sa);
-            else hipLaunchKernelGGL((elem_single_persistent<float, 1, R>), grid, block, 0, st, sa);
-        }
+        nel = std::min(nel, per_cu * std::max(ncu, 1));
+    }
+    grid = dim3(nel);
+    return 0;
+}
+
+// The fused kernel: 64 rows and 16 bubbles when the batch's bounds allow it.
+// The pools are the smallest that hold every element in one of the modes, the
+// waves those that fill a CU with the workgroups that the pools let in
+// (workgroups x waves, 13,824 H1 p = 3 elements in FP64): 3 x 4 0.46 ms, 4 x 4
+// at 128 registers 0.46, 4 x 3 at 168 registers 0.45, 4 x 2 0.49, 4 x 1 0.56.
+// 8,000 H1 p = 4 elements: 2 x 8 at 128 registers 0.78 ms in FP64 and 0.68 in
+// FP32, 2 x 4 at 256 0.78 and 0.73; 6 waves at 168 registers leave a CU one
+// workgroup (a SIMD would have to take four of their waves): 1.1.
+// 8,000 H(curl) p = 2 elements: 3 x 4 0.30 ms, 2 x 4 0.42.
+template <typename T>
+static int launch_fused(int space, const ElemArgs &args, const CondArgs &cd, int max_ndof, int max_nbubble,
+                        hipStream_t st)
+{
+    const bool small = max_ndof <= BR / 2 && max_nbubble <= NBF / 2;
+    dim3 grid;
+    const SingleArgs sa{args, cd};
+    if (int r = fused_grid(args.nel, space == HP3D_H1 ? (small ? 4 : 2) : (small ? 3 : 1), grid)) return r;
+    if (space == HP3D_H1) {
+        if (small) hipLaunchKernelGGL((sf_fused_kernel<T, 0, 64, 1, 3, 4500, 3>), grid, dim3(192), 0, st, sa);
+        else hipLaunchKernelGGL((sf_fused_kernel<T, 0, 128, 2, 8, 8352, 4>), grid, dim3(512), 0, st, sa);
     } else {
-        dim3 grid(args.nel);
-        if (space == HP3D_H1) {
-            if (precision == HP3D_FP64) hipLaunchKernelGGL((elem_single_kernel<double, 0, R>), grid, block, 0, st, args, cd);
-            else hipLaunchKernelGGL((elem_single_kernel<float, 0, R>), grid, block, 0, st, args, cd);
-        } else {
-            if (precision == HP3D_FP64) hipLaunchKernelGGL((elem_single_kernel<double, 1, R>), grid, block, 0, st, args, cd);
-            else hipLaunchKernelGGL((elem_single_kernel<float, 1, R>), grid, block, 0, st, args, cd);
-        }
+        if (small) hipLaunchKernelGGL((sf_fused_kernel<T, 1, 64, 1, 4, 5660, 3>), grid, dim3(256), 0, st, sa);
+        else hipLaunchKernelGGL((sf_fused_kernel<T, 1, 128, 2, 8, 13932, 2>), grid, dim3(512), 0, st, sa);
     }
     HIPCHK(hipGetLastError());
     return 0;
 }
 
-// the single-block kernel for a batch whose elements have at most max_ndof
-// dofs and (when condensing) at most max_nbubble bubbles: 64 rows when they fit
+// the single-launch path of a batch whose elements have at most max_ndof
+// (<= 128) dofs and max_nbubble (<= 32) bubbles
 static int launch_single(int space, int precision, const ElemArgs &args, const CondArgs &cd,
                          int max_ndof, int max_nbubble, hipStream_t st)
 {
+    if (precision == HP3D_FP64) return launch_fused<double>(space, args, cd, max_ndof, max_nbubble, st);
+    if (precision == HP3D_FP32) return launch_fused<float>(space, args, cd, max_ndof, max_nbubble, st);
     if (max_ndof <= BR / 2 && (cd.aii == nullptr || max_nbubble <= NBF / 2))
-        return launch_single_r<BR / 2>(space, precision, args, cd, st);
-    return launch_single_r<BR>(space, precision, args, cd, st);
+        return launch_single_bf16<BR / 2>(space, args, cd, st);
+    return launch_single_bf16<BR>(space, args, cd, st);
 }
 
 // the sum-factorised element kernel; few elements are split over several
@@ -2692,12 +2679,12 @@ static int launch_sf(int space, const ElemArgs &args, int max_ndof, hipStream_t 
 static int launch_elem(int space, int precision, const ElemArgs &args, int max_ndof,
                        hipStream_t st)
 {
+    if (precision == HP3D_FP64) return launch_sf<double>(space, args, max_ndof, st);
+    if (precision == HP3D_FP32) return launch_sf<float>(space, args, max_ndof, st);
     if (max_ndof <= BR) {
         CondArgs cd{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
         return launch_single(space, precision, args, cd, max_ndof, 0, st);
     }
-    if (precision == HP3D_FP64) return launch_sf<double>(space, args, max_ndof, st);
-    if (precision == HP3D_FP32) return launch_sf<float>(space, args, max_ndof, st);
     // the BF16 trial: geometry pass, then the block-tiled MFMA kernel
     if (!args.gws) return HP3D_E_ARG;
     dim3 grid(args.nel, nblocks_for(max_ndof)), block(WGE);

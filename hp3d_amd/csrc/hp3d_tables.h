@@ -486,9 +486,8 @@ constexpr int ROW_NEG = 1 << 14; // sign bit of dof_row
 // product, or -1 when the element has no such dof
 HP3D_HD inline int dof_row(int space, int a, int i0, int i1, int i2, const ElemOrders &o, const DofBases &b)
 {
-    const int ix[3] = {i0, i1, i2};
     if (space == 0) a = -1;
-    else if (ix[a] < 1) return -1;
+    else if ((a == 0 ? i0 : a == 1 ? i1 : i2) < 1) return -1;
     // directions in which the dof is not one of the two affine functions
     const bool in0 = a == 0 || i0 >= 2, in1 = a == 1 || i1 >= 2, in2 = a == 2 || i2 >= 2;
     const int inner = (int)in0 + (int)in1 + (int)in2;
@@ -533,11 +532,11 @@ HP3D_HD inline int dof_row(int space, int a, int i0, int i1, int i2, const ElemO
 }
 
 // 1D tables of the sum-factorised kernels at the n Gauss points of a
-// direction: f[n][0][i][q] = chi_i(x_q), f[n][1][i][q] = chi_i'(x_q), and the
-// weights of the rule on [0, 1]
+// direction: f[n][0][i][q] = chi_i(x_q), f[n][1][i][q] = chi_i'(x_q), the
+// weights w of the rule on [0, 1], and g = chi_0 - 1/2
 struct SfTables {
     double f[MAXP + 2][2][MAXP + 1][8];
-    double w[MAXP + 2][8];
+    double w[MAXP + 2][8], g[MAXP + 2][8];
 };
 constexpr SfTables make_sf_tables()
 {
@@ -558,6 +557,7 @@ constexpr SfTables make_sf_tables()
                 t.f[n][1][i][q] = p[i - 1];
             }
             t.w[n][q] = 0.5 * gw[n - 1][q];
+            t.g[n][q] = -0.5 * gx[n - 1][q];
         }
     return t;
 }

@@ -70,3 +70,70 @@ def test_anisotropic(gpu, space, porder):
     m = mesh.structured((2, 1, 1), porder=porder, perturb=0.0, perm_seed=3 + sum(porder), coef=[0.7, 1.9])
     x = m.xnod() + 0.05 * np.random.default_rng(sum(porder)).uniform(-1, 1, (2, 8, 3))
     check(space, m.norder, m.nori_e, m.nori_f, x, m.coef)
+
+
+def condensed_against_oracle(space, no, oe, of, xnod, coef, rules, precision=0):
+    """celem of one launch against the oracle (FP64: Aii and Bi 1e-12, the
+    bubble solutions nb cond(Abb) eps; FP32 K only rounds K)."""
+    import torch
+
+    import hp3d_amd
+    from test_gpu_elem import TOL64, compare
+
+    load = oracle.LOAD_SINSINSIN if space == 0 else oracle.LOAD_CURL_SIN
+    batch = hp3d_amd.ElementBatch(space, no, oe, of, xnod, coef, load=load, rules=rules)
+    assert batch.bin_paths == ["fused"]
+    out = batch.alloc_outputs(precision)
+    for v in out.values():
+        v.fill_(float("nan"))
+    batch.celem(out, precision)
+    bare = batch.run(precision, want_k=False)
+    torch.cuda.synchronize()
+    assert (batch.check_status() == 0).all()
+    ref = oracle.element_loop(space, no, oe, of, xnod, coef, load, ldk=int(batch.n.max()), herm=True)
+    compare(batch, out, ref, TOL64 if precision == 0 else 1e-7, TOL64)
+    for e in range(batch.nel):
+        k = batch.k_of(out, e)
+        assert np.array_equal(k, k.T)
+        a, b = batch.aii_of(out, e), batch.aii_of(bare, e)
+        assert np.array_equal(a, a.T) and np.array_equal(a, b)
+        ni = int(batch.ni[e])
+        if batch.nb[e] == 0:
+            assert rel(a, ref["k"][e].T[:ni, :ni]) < TOL64
+            assert np.array_equal(batch.vec_of(out, "bi", e, ni), batch.vec_of(out, "b", e))
+
+
+FUSED = ({"max_ndof": 128, "max_nbubble": 32, "path": "fused"}, {"path": "two_pass"})
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("space", [0, 1])
+@pytest.mark.parametrize("most", [(64, 16), (128, 32)])
+def test_fused_any_codes(gpu, space, most, precision):
+    """Interior orders of at most 3 under edges and faces of up to 6: every
+    storage mode of the one-launch kernel, the streamed one (seven functions in
+    each direction) among them."""
+    rng = np.random.default_rng(70 + space + most[0])
+    no, oe, of = random_codes(rng, 4000, 6)
+    b = rng.integers(1, 4 if space == 0 else 3, (4000, 3))
+    no[:, 18] = 100 * b[:, 0] + 10 * b[:, 1] + b[:, 2]
+    flat = rng.random(4000) < 0.8     # faces of order 1: mostly edges
+    no[flat, 12:18] = 11
+    from hp3d_amd.elem import ndof, nquad
+
+    n, nb = ndof(space, no)
+    ok = np.nonzero((n <= most[0]) & (nb <= most[1]) & (n > (0 if most[0] == 64 else 64)))[0]
+    q = nquad(no[ok], of[ok]).min(1)
+    pick = np.concatenate([ok[q == 7][:10], ok[q < 7][:14]])
+    assert pick.size >= 16
+    v = mesh.VERT_XYZ[None] + 0.15 * rng.uniform(-1, 1, (pick.size, 8, 3))
+    condensed_against_oracle(space, no[pick], oe[pick], of[pick], v, rng.uniform(0.5, 2.0, pick.size), FUSED, precision)
+
+
+@pytest.mark.parametrize("space,porder", [(0, (1, 1, 1)), (0, (2, 1, 2)), (0, (4, 4, 4)), (0, (3, 5, 4)), (0, (5, 4, 3)),
+                                          (0, (6, 2, 2)), (0, (2, 6, 5)), (0, (6, 4, 2)), (0, (3, 3, 6)), (0, (1, 6, 6)),
+                                          (1, (1, 1, 1)), (1, (2, 2, 2)), (1, (3, 3, 2)), (1, (1, 5, 2)), (1, (6, 1, 1))])
+def test_fused_anisotropic(gpu, space, porder):
+    m = mesh.structured((2, 1, 1), porder=porder, perm_seed=5 + sum(porder), coef=[0.7, 1.9])
+    x = m.xnod() + 0.05 * np.random.default_rng(sum(porder)).uniform(-1, 1, (2, 8, 3))
+    condensed_against_oracle(space, m.norder, m.nori_e, m.nori_f, x, m.coef, FUSED)
