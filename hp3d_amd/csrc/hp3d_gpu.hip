@@ -2219,288 +2219,6 @@ __global__ __launch_bounds__(WG) void dirichlet_lift_kernel(LiftArgs a)
     }
 }
 
-// ------------------------------------------------------- field evaluation
-//
-// One workgroup per element evaluates finite-element fields from element dof
-// vectors at the quadrature points (soleval, element/util/soleval.F90, with
-// the dofs in element order) and integrates one of:
-//   HP3D_FIELD_ERROR    element_error (element/util/compute_error.F90:226-400):
-//                       set_3Dint rule with INTEGRATION = 2; out[2e] = errorH
-//                       (int |grad(u - u_h)|^2 + |u - u_h|^2) or errorE (curl
-//                       and value), out[2e+1] = the same norm of the exact u
-//   HP3D_FIELD_ADJOINT  out[e] = -coef_e int grad v_h . grad u_h (H1) or
-//                       -coef_e int v_h . u_h (H(curl)): lambda_e^T (dK_e /
-//                       dlog coef_e) u_e with a minus sign, i.e. dJ/dtheta_e
-//                       for coef = exp(theta), recomputed at the points of the
-//                       element rule without forming K_e
-//   HP3D_FIELD_L2       out[e] = int u_h . u_h and r[off_v[e] + k] = int
-//                       phi_k . u_h (the element mass matrix times u_e)
-// Threads own quadrature points; the dof loop reads descriptors and
-// coefficients from LDS (same address across the wave: broadcast).
-
-struct FieldArgs {
-    int space, mode, nel, ngeo, exact;
-    const int *norder, *nori_e, *nori_f;
-    const double *xnod, *coef;
-    const long long *off_v;
-    const double *u, *v;
-    double *out, *r;
-    int *status;
-};
-
-// exact solutions of the manufactured problems (value, gradient); the
-// selector is the load selector of the same problem
-__device__ inline void exact_h1(int sel, const double *x, double &u, double *du)
-{
-    const double pi = 3.14159265358979323846;
-    u = du[0] = du[1] = du[2] = 0.0;
-    if (sel == HP3D_LOAD_SINSINSIN) {
-        double sx = sin(pi * x[0]), sy = sin(pi * x[1]), sz = sin(pi * x[2]);
-        u = sx * sy * sz;
-        du[0] = pi * cos(pi * x[0]) * sy * sz;
-        du[1] = pi * sx * cos(pi * x[1]) * sz;
-        du[2] = pi * sx * sy * cos(pi * x[2]);
-    } else if (sel == HP3D_LOAD_CONV) {
-        double sx = sin(pi * x[0]), sh = sinh(pi * x[1]), z2 = x[2] * x[2];
-        u = sx * sh * z2;
-        du[0] = pi * cos(pi * x[0]) * sh * z2;
-        du[1] = pi * sx * cosh(pi * x[1]) * z2;
-        du[2] = 2.0 * sx * sh * x[2];
-    } else if (sel == HP3D_LOAD_POLY2) {
-        double a0 = x[0] * (1.0 - x[0]), a1 = x[1] * (1.0 - x[1]), a2 = x[2] * (1.0 - x[2]);
-        u = a0 * a1 * a2;
-        du[0] = (1.0 - 2.0 * x[0]) * a1 * a2;
-        du[1] = a0 * (1.0 - 2.0 * x[1]) * a2;
-        du[2] = a0 * a1 * (1.0 - 2.0 * x[2]);
-    } else if (sel == HP3D_LOAD_XYZ) {
-        u = x[0] * x[1] * x[2];
-        du[0] = x[1] * x[2];
-        du[1] = x[0] * x[2];
-        du[2] = x[0] * x[1];
-    }
-}
-
-__device__ inline void exact_hcurl(int sel, const double *x, double *e, double *curl)
-{
-    const double pi = 3.14159265358979323846;
-    for (int i = 0; i < 3; ++i) e[i] = curl[i] = 0.0;
-    if (sel == HP3D_LOAD_CURL_SIN) {
-        e[0] = sin(pi * x[1]) * sin(pi * x[2]);
-        curl[1] = pi * sin(pi * x[1]) * cos(pi * x[2]);
-        curl[2] = -pi * cos(pi * x[1]) * sin(pi * x[2]);
-    }
-}
-
-// set_3Dint brick rule (set_3D_int.F90:8-21,203-244): face orders as coded
-// (no swap), orders raised by INTEGRATION and capped at MAXP
-__device__ inline void quad_counts_plain(const ElemOrders &o, int integration, int nq[3])
-{
-    int m[3] = {o.b[0], o.b[1], o.b[2]};
-    for (int e = 0; e < 12; ++e) {
-        int d = edge_t(e).dir;
-        m[d] = o.pe[e] > m[d] ? o.pe[e] : m[d];
-    }
-    for (int f = 0; f < 6; ++f) {
-        FaceT ft = face_t(f);
-        m[ft.ax0] = o.fh[f] > m[ft.ax0] ? o.fh[f] : m[ft.ax0];
-        m[ft.ax1] = o.fv[f] > m[ft.ax1] ? o.fv[f] : m[ft.ax1];
-    }
-    for (int d = 0; d < 3; ++d) {
-        int q = m[d] + integration;
-        nq[d] = (q < MAXP ? q : MAXP) + 1;
-    }
-}
-
-// reference-coordinate value and gradient of the scalar dof d at point p
-__device__ __forceinline__ void dof_ref(unsigned d, Pt p, const double (*tv)[NTAB * NPT],
-                                        const double (*td)[NTAB * NPT], double &ph, double gr[3])
-{
-    int i0 = desc_ix(d, 0), i1 = desc_ix(d, 1), i2 = desc_ix(d, 2);
-    double v0 = tv[0][p.l1 * NTAB + i0], v1 = tv[1][p.l2 * NTAB + i1], v2 = tv[2][p.l3 * NTAB + i2];
-    double d0 = td[0][p.l1 * NTAB + i0], d1 = td[1][p.l2 * NTAB + i1], d2 = td[2][p.l3 * NTAB + i2];
-    ph = v0 * v1 * v2;
-    gr[0] = d0 * v1 * v2;
-    gr[1] = v0 * d1 * v2;
-    gr[2] = v0 * v1 * d2;
-}
-
-// field of coefficients c at point p in reference form: H1 value f[0] and
-// gradient g; H(curl) E_ref in f[0..2] and curl_ref in g
-template <int SPACE>
-__device__ __forceinline__ void eval_ref(int n, const unsigned *dsc, const double *c, Pt p,
-                                         const double (*tv)[NTAB * NPT], const double (*td)[NTAB * NPT],
-                                         double f[3], double g[3])
-{
-    for (int i = 0; i < 3; ++i) f[i] = g[i] = 0.0;
-    for (int k = 0; k < n; ++k) {
-        unsigned d = dsc[k];
-        double ph, gr[3];
-        dof_ref(d, p, tv, td, ph, gr);
-        double ck = c[k];
-        if (SPACE == 0) {
-            f[0] += ck * ph;
-            for (int i = 0; i < 3; ++i) g[i] += ck * gr[i];
-        } else {
-            int cp = desc_comp(d);
-            double sg = desc_neg(d) ? -ck : ck;
-            // E = s phi e_cp, curl E = s grad(phi) x e_cp
-            f[cp] += sg * ph;
-            g[(cp + 1) % 3] += sg * gr[(cp + 2) % 3];
-            g[(cp + 2) % 3] -= sg * gr[(cp + 1) % 3];
-        }
-    }
-}
-
-// physical value / gradient (H1) or E / curl E (H(curl)) from the reference form
-template <int SPACE>
-__device__ __forceinline__ void to_phys(const double f[3], const double g[3], double jm[3][3], double inv[3][3],
-                                        double det, double fp[3], double gp[3])
-{
-    if (SPACE == 0) {
-        fp[0] = f[0];
-        fp[1] = fp[2] = 0.0;
-        for (int j = 0; j < 3; ++j) gp[j] = g[0] * inv[0][j] + g[1] * inv[1][j] + g[2] * inv[2][j];
-    } else {
-        for (int j = 0; j < 3; ++j) {
-            fp[j] = f[0] * inv[0][j] + f[1] * inv[1][j] + f[2] * inv[2][j];
-            gp[j] = (jm[j][0] * g[0] + jm[j][1] * g[1] + jm[j][2] * g[2]) / det;
-        }
-    }
-}
-
-template <int SPACE>
-__global__ __launch_bounds__(WG) void field_kernel(FieldArgs a)
-{
-    constexpr int MAXN = SPACE == 0 ? MAXN_H1 : MAXN_E;
-    __shared__ ElemShared es;
-    __shared__ double tv[3][NTAB * NPT], td[3][NTAB * NPT];
-    __shared__ unsigned dsc[MAXN];
-    __shared__ unsigned dgeo[MAXN_H1];
-    __shared__ double cu[MAXN], cv[MAXN];
-    __shared__ double pw[3 * MAXQ];
-    __shared__ double red[2][WG / 64];
-
-    const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) {
-        ElemShared s;
-        s.ok = decode_orders(a.norder + 19 * (size_t)e, a.nori_e + 12 * (size_t)e,
-                             a.nori_f + 6 * (size_t)e, s.o);
-        s.n = s.nb = s.nint = s.nh = 0;
-        s.nq[0] = s.nq[1] = s.nq[2] = 1;
-        if (s.ok) {
-            dof_counts(SPACE, s.o, s.n, s.nb);
-            int nbh;
-            dof_counts(0, s.o, s.nh, nbh);
-            if (a.mode == HP3D_FIELD_ERROR) quad_counts_plain(s.o, 2, s.nq);
-            else quad_counts(s.o, s.nq);
-            s.nint = s.nq[0] * s.nq[1] * s.nq[2];
-            if (a.ngeo > s.nh) s.ok = 0;
-        }
-        s.negjac = 0;
-        es = s;
-    }
-    __syncthreads();
-    if (!es.ok) {
-        if (tid == 0 && a.status) a.status[e] = HP3D_E_ORDER;
-        return;
-    }
-    const int n = es.n, nint = es.nint;
-    if (wave < 3) fill_tables(es.nq[wave], tv[wave], td[wave]);
-    const double *ue = a.u + a.off_v[e];
-    const double *ve = a.mode == HP3D_FIELD_ADJOINT ? a.v + a.off_v[e] : nullptr;
-    const ElemOrders ol = es.o; // in registers for the descriptor walks
-    for (int k = tid; k < n; k += WG) {
-        dsc[k] = SPACE == 0 ? desc_h1(k, ol) : desc_hcurl(k, ol);
-        cu[k] = ue[k];
-        if (ve) cv[k] = ve[k];
-    }
-    for (int k = tid; k < a.ngeo; k += WG) dgeo[k] = desc_h1(k, es.o);
-    __syncthreads();
-
-    const double *xn = a.xnod + 3 * (size_t)a.ngeo * e;
-    const double coef = a.coef ? a.coef[e] : 1.0;
-    double acc0 = 0.0, acc1 = 0.0;
-    bool neg = false;
-    for (int l = tid; l < nint; l += WG) {
-        Pt p = point_ix(l, es.nq);
-        double x[3], jm[3][3], inv[3][3], det, w;
-        point_map(p, es.nq, tv, td, dgeo, xn, a.ngeo, x, jm, inv, det, w);
-        neg = neg || det < 0.0;
-        const double wd = w * det;
-        double f[3], g[3], fu[3], gu[3];
-        eval_ref<SPACE>(n, dsc, cu, p, tv, td, f, g);
-        to_phys<SPACE>(f, g, jm, inv, det, fu, gu);
-        if (a.mode == HP3D_FIELD_ERROR) {
-            double fe[3], ge[3];
-            if (SPACE == 0) {
-                exact_h1(a.exact, x, fe[0], ge);
-                fe[1] = fe[2] = 0.0;
-            } else {
-                exact_hcurl(a.exact, x, fe, ge);
-            }
-            for (int j = 0; j < 3; ++j) {
-                acc0 += ((ge[j] - gu[j]) * (ge[j] - gu[j]) + (fe[j] - fu[j]) * (fe[j] - fu[j])) * wd;
-                acc1 += (ge[j] * ge[j] + fe[j] * fe[j]) * wd;
-            }
-        } else if (a.mode == HP3D_FIELD_ADJOINT) {
-            double fv[3], gv[3];
-            eval_ref<SPACE>(n, dsc, cv, p, tv, td, f, g);
-            to_phys<SPACE>(f, g, jm, inv, det, fv, gv);
-            if (SPACE == 0) acc0 -= coef * (gu[0] * gv[0] + gu[1] * gv[1] + gu[2] * gv[2]) * wd;
-            else acc0 -= coef * (fu[0] * fv[0] + fu[1] * fv[1] + fu[2] * fv[2]) * wd;
-        } else {
-            acc0 += (fu[0] * fu[0] + fu[1] * fu[1] + fu[2] * fu[2]) * wd;
-            // weighted field pulled back to reference components: phi_k . u_h w det
-            if (SPACE == 0) {
-                pw[l] = fu[0] * wd;
-            } else {
-                for (int i = 0; i < 3; ++i)
-                    pw[3 * l + i] = (inv[i][0] * fu[0] + inv[i][1] * fu[1] + inv[i][2] * fu[2]) * wd;
-            }
-        }
-    }
-    if (neg) es.negjac = 1;
-    // workgroup sums
-    for (int off = 32; off > 0; off >>= 1) {
-        acc0 += __shfl_down(acc0, off);
-        acc1 += __shfl_down(acc1, off);
-    }
-    if (lane == 0) {
-        red[0][wave] = acc0;
-        red[1][wave] = acc1;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        double s0 = 0.0, s1 = 0.0;
-        for (int w = 0; w < WG / 64; ++w) {
-            s0 += red[0][w];
-            s1 += red[1][w];
-        }
-        if (a.mode == HP3D_FIELD_ERROR) {
-            a.out[2 * (size_t)e] = s0;
-            a.out[2 * (size_t)e + 1] = s1;
-        } else {
-            a.out[e] = s0;
-        }
-        if (a.status) a.status[e] = es.negjac ? HP3D_NEG_JACOBIAN : 0;
-    }
-    if (a.mode == HP3D_FIELD_L2 && a.r) {
-        double *re = a.r + a.off_v[e];
-        for (int k = tid; k < n; k += WG) {
-            unsigned d = dsc[k];
-            double s = 0.0;
-            for (int l = 0; l < nint; ++l) {
-                Pt p = point_ix(l, es.nq);
-                double ph, gr[3];
-                dof_ref(d, p, tv, td, ph, gr);
-                if (SPACE == 0) s += ph * pw[l];
-                else s += (desc_neg(d) ? -ph : ph) * pw[3 * l + desc_comp(d)];
-            }
-            re[k] = s;
-        }
-    }
-}
-
 // Segmented gather-sum: out[t] = sum over j in [ptr[t], ptr[t+1]) of in[src[j]].
 // With src listing, for every nonzero of a global matrix (or entry of a global
 // vector), the positions of its element contributions in the packed condensed
@@ -3140,8 +2858,14 @@ int hp3d_gpu_field_batch(int space, int mode, int nel, const int *norder, const 
     FieldArgs a{space, mode, nel, ngeo, exact, norder, nori_e, nori_f, xnod, coef, off_v, u, v,
                 out, r, status};
     hipStream_t st = (hipStream_t)stream;
-    if (space == HP3D_H1) hipLaunchKernelGGL(field_kernel<0>, dim3(nel), dim3(WG), 0, st, a);
-    else hipLaunchKernelGGL(field_kernel<1>, dim3(nel), dim3(WG), 0, st, a);
+    const dim3 grid(nel), block(128);
+    if (mode == HP3D_FIELD_ADJOINT) {
+        if (space == HP3D_H1) hipLaunchKernelGGL((field_kernel<0, true>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((field_kernel<1, true>), grid, block, 0, st, a);
+    } else {
+        if (space == HP3D_H1) hipLaunchKernelGGL((field_kernel<0, false>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((field_kernel<1, false>), grid, block, 0, st, a);
+    }
     HIPCHK(hipGetLastError());
     return 0;
 }

@@ -168,7 +168,7 @@ __device__ __forceinline__ bool sf_setup(const ElemArgs &a, int e, SfElem &es, d
         const int k = tid + i * WGS;
         xv[i] = 0.0;
         if (k < nx) xv[i] = a.xnod[(size_t)3 * a.ngeo * e + k];
-        else if (k == 3 * XS_MAX) xv[i] = a.coef[e];
+        else if (k == 3 * XS_MAX) xv[i] = a.coef ? a.coef[e] : 1.0;
     }
     if (tid < 64) {
         int v = 0;
@@ -247,31 +247,31 @@ __device__ __forceinline__ bool sf_setup(const ElemArgs &a, int e, SfElem &es, d
     return es.ok != 0;
 }
 
+// the value of a role
+__device__ __forceinline__ int sf_pick(int role, int b, int a, int c) { return role == 0 ? b : role == 1 ? a : c; }
+
 // 1D tables of the three directions in LDS
 struct SfTab {
     double f[3][2][SF_I * 8];
     double w[3][8];
 };
 template <int WGS>
-__device__ __forceinline__ void sf_fill_tab(const SfElem &es, SfTab &t, int tid)
+__device__ __forceinline__ void sf_fill_tab(const int (&m)[3], SfTab &t, int tid)
 {
     constexpr int LEN = 2 * SF_I * 8, NL = (3 * LEN + WGS - 1) / WGS;
     double v[NL];
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
         const int k = min(tid + i * WGS, 3 * LEN - 1), d = k / LEN;
-        v[i] = (&c_sf.f[es.m[d]][0][0][0])[k - d * LEN];
+        v[i] = (&c_sf.f[sf_pick(d, m[0], m[1], m[2])][0][0][0])[k - d * LEN];
     }
     const int dw = min(tid >> 3, 2);
-    const double w = c_sf.w[es.m[dw]][tid & 7];
+    const double w = c_sf.w[sf_pick(dw, m[0], m[1], m[2])][tid & 7];
 #pragma unroll
     for (int i = 0; i < NL; ++i)
         if (tid + i * WGS < 3 * LEN) (&t.f[0][0][0])[tid + i * WGS] = v[i];
     if (tid < 24) t.w[dw][tid & 7] = w;
 }
-
-// the value of a role
-__device__ __forceinline__ int sf_pick(int role, int b, int a, int c) { return role == 0 ? b : role == 1 ? a : c; }
 
 // dof rows by 1D indexes: row[((comp * 7 + iA) * 7 + iB) * 8 + iC], iA < m[1],
 // iB < m[0]
@@ -302,10 +302,67 @@ __device__ __forceinline__ void sf_fill_gmap(const SfElem &es, int ngeo, unsigne
     }
 }
 
+// The map at the point with 1D indexes (q0, q1, q2) in x, y and z
+// (geom3D.F90:77-91, geom.F90:57-113): x, J (jm[c][i] = d x_c / d xi_i), its
+// inverse [reference, physical] and det J.
+template <bool STAGED>
+__device__ __forceinline__ double sf_map(const SfElem &es, const SfTab &tb, const unsigned short *gmap,
+                                         const double *xn, int ngeo, int q0, int q1, int q2, double (&x)[3],
+                                         double (&jm)[3][3], double (&inv)[3][3])
+{
+    const int r0 = es.rol[0], r1 = es.rol[1], r2 = es.rol[2]; // roles of x, y, z
+#pragma unroll
+    for (int c = 0; c < 3; ++c) x[c] = jm[c][0] = jm[c][1] = jm[c][2] = 0.0;
+    auto node = [&](const double *xk, double v0, double v1, double v2, double g0, double g1, double g2) {
+        const double ph = v0 * v1 * v2, h0 = g0 * v1 * v2, h1 = v0 * g1 * v2, h2 = v0 * v1 * g2;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const double xc = xk[c];
+            x[c] += xc * ph;
+            jm[c][0] += xc * h0;
+            jm[c][1] += xc * h1;
+            jm[c][2] += xc * h2;
+        }
+    };
+    if (STAGED && ngeo == 8) {
+        double v[3][2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            v[0][i] = tb.f[r0][0][8 * i + q0];
+            v[1][i] = tb.f[r1][0][8 * i + q1];
+            v[2][i] = tb.f[r2][0][8 * i + q2];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int i0 = vtx_mu(k, 0), i1 = vtx_mu(k, 1), i2 = vtx_mu(k, 2);
+            node(xn + 3 * k, v[0][i0], v[1][i1], v[2][i2], i0 ? 1.0 : -1.0, i1 ? 1.0 : -1.0, i2 ? 1.0 : -1.0);
+        }
+    } else {
+        for (int k = 0; k < ngeo; ++k) {
+            const int g = gmap[k], i0 = 8 * (g & 7) + q0, i1 = 8 * ((g >> 3) & 7) + q1, i2 = 8 * ((g >> 6) & 7) + q2;
+            const double sg = g & 512 ? -1.0 : 1.0;
+            node(xn + 3 * k, sg * tb.f[r0][0][i0], tb.f[r1][0][i1], tb.f[r2][0][i2], sg * tb.f[r0][1][i0],
+                 tb.f[r1][1][i1], tb.f[r2][1][i2]);
+        }
+    }
+    const double c00 = jm[1][1] * jm[2][2] - jm[2][1] * jm[1][2], c01 = jm[2][1] * jm[0][2] - jm[0][1] * jm[2][2],
+                 c02 = jm[0][1] * jm[1][2] - jm[1][1] * jm[0][2];
+    const double det = jm[0][0] * c00 + jm[1][0] * c01 + jm[2][0] * c02;
+    const double rdet = 1.0 / det;
+    inv[0][0] = c00 * rdet;
+    inv[0][1] = c01 * rdet;
+    inv[0][2] = c02 * rdet;
+    inv[1][0] = (jm[2][0] * jm[1][2] - jm[1][0] * jm[2][2]) * rdet;
+    inv[1][1] = (jm[0][0] * jm[2][2] - jm[2][0] * jm[0][2]) * rdet;
+    inv[1][2] = (jm[1][0] * jm[0][2] - jm[0][0] * jm[1][2]) * rdet;
+    inv[2][0] = (jm[1][0] * jm[2][1] - jm[2][0] * jm[1][1]) * rdet;
+    inv[2][1] = (jm[2][0] * jm[0][1] - jm[0][0] * jm[2][1]) * rdet;
+    inv[2][2] = (jm[0][0] * jm[1][1] - jm[1][0] * jm[0][1]) * rdet;
+    return det;
+}
+
 // Metric fields and load of every quadrature point, q = (qA mB + qB) mC + qC,
-// field f at d[f * nint + q]: the map, its Jacobian and inverse as in
-// point_map, with the weights folded in (geom3D.F90:77-91, geom.F90:57-113,
-// elem_opt.F90:101-122).  Returns true when a point of this thread has det < 0.
+// field f at d[f * nint + q], the weights folded in (elem_opt.F90:101-122).  Returns true when a point of this thread has det < 0.
 // The load and the metric of a point are evaluated by different waves, side by
 // side (the lower half of the workgroup has the metric).
 template <int SPACE, bool STAGED>
@@ -323,54 +380,10 @@ __device__ __forceinline__ bool sf_points_of(const SfElem &es, const SfTab &tb, 
     for (int l = tid; l < Q; l += wgs) {
         const int l1 = div_small(l, mC), qC = l - l1 * mC, qA = div_small(l1, mB), qB = l1 - qA * mB;
         const int q0 = sf_pick(r0, qB, qA, qC), q1 = sf_pick(r1, qB, qA, qC), q2 = sf_pick(r2, qB, qA, qC);
-        double x[3] = {0.0, 0.0, 0.0}, jm[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
-        auto node = [&](const double *xk, double v0, double v1, double v2, double g0, double g1, double g2) {
-            const double ph = v0 * v1 * v2, h0 = g0 * v1 * v2, h1 = v0 * g1 * v2, h2 = v0 * v1 * g2;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const double xc = xk[c];
-                x[c] += xc * ph;
-                jm[c][0] += xc * h0;
-                jm[c][1] += xc * h1;
-                jm[c][2] += xc * h2;
-            }
-        };
-        if (STAGED && ngeo == 8) {
-            double v[3][2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                v[0][i] = tb.f[r0][0][8 * i + q0];
-                v[1][i] = tb.f[r1][0][8 * i + q1];
-                v[2][i] = tb.f[r2][0][8 * i + q2];
-            }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int i0 = vtx_mu(k, 0), i1 = vtx_mu(k, 1), i2 = vtx_mu(k, 2);
-                node(xn + 3 * k, v[0][i0], v[1][i1], v[2][i2], i0 ? 1.0 : -1.0, i1 ? 1.0 : -1.0, i2 ? 1.0 : -1.0);
-            }
-        } else {
-            for (int k = 0; k < ngeo; ++k) {
-                const int g = gmap[k], i0 = 8 * (g & 7) + q0, i1 = 8 * ((g >> 3) & 7) + q1, i2 = 8 * ((g >> 6) & 7) + q2;
-                const double sg = g & 512 ? -1.0 : 1.0;
-                node(xn + 3 * k, sg * tb.f[r0][0][i0], tb.f[r1][0][i1], tb.f[r2][0][i2], sg * tb.f[r0][1][i0],
-                     tb.f[r1][1][i1], tb.f[r2][1][i2]);
-            }
-        }
-        const double c00 = jm[1][1] * jm[2][2] - jm[2][1] * jm[1][2], c01 = jm[2][1] * jm[0][2] - jm[0][1] * jm[2][2],
-                     c02 = jm[0][1] * jm[1][2] - jm[1][1] * jm[0][2];
-        const double det = jm[0][0] * c00 + jm[1][0] * c01 + jm[2][0] * c02;
+        double x[3], jm[3][3], inv[3][3];
+        const double det = sf_map<STAGED>(es, tb, gmap, xn, ngeo, q0, q1, q2, x, jm, inv);
         neg = neg || det < 0.0;
         const double rdet = 1.0 / det;
-        double inv[3][3];
-        inv[0][0] = c00 * rdet;
-        inv[0][1] = c01 * rdet;
-        inv[0][2] = c02 * rdet;
-        inv[1][0] = (jm[2][0] * jm[1][2] - jm[1][0] * jm[2][2]) * rdet;
-        inv[1][1] = (jm[0][0] * jm[2][2] - jm[2][0] * jm[0][2]) * rdet;
-        inv[1][2] = (jm[1][0] * jm[0][2] - jm[0][0] * jm[1][2]) * rdet;
-        inv[2][0] = (jm[1][0] * jm[2][1] - jm[2][0] * jm[1][1]) * rdet;
-        inv[2][1] = (jm[2][0] * jm[0][1] - jm[0][0] * jm[2][1]) * rdet;
-        inv[2][2] = (jm[0][0] * jm[1][1] - jm[1][0] * jm[0][1]) * rdet;
         const double wd = det * (tb.w[0][qB] * tb.w[1][qA] * tb.w[2][qC]);
         if (half || wl == 0) {
             double f[3];
@@ -1090,12 +1103,11 @@ __device__ __forceinline__ void sf_matrix(const SfElem &es, const SfTab &tb, con
 // Load vector, entry by entry as put(row, value): the load fields transformed
 // in place, one direction after the other; ends with a barrier.
 template <int SPACE, int WGS, typename PUT>
-__device__ __forceinline__ void sf_load(const SfElem &es, const SfTab &tb, const short *row, double *d, const PUT &put,
+__device__ __forceinline__ void sf_load(const SfElem &es, const SfTab &tb, const short *row, double *g, const PUT &put,
                                         int tid)
 {
     constexpr int U = (sf_comps(SPACE) * SF_I * SF_I * SF_I + WGS - 1) / WGS;
     const int mA = es.m[1], mB = es.m[0], mC = es.m[2], Q = es.nint, len = sf_comps(SPACE) * Q;
-    double *const g = d + (SPACE == 0 ? 6 : 12) * Q;
 #pragma unroll
     for (int step = 0; step < 3; ++step) {
         double v[U];
@@ -1147,7 +1159,7 @@ __global__ __launch_bounds__(WGS, WPE) void sf_elem_kernel(ElemArgs a)
         if (tid == 0 && part == 0 && a.status) a.status[e] = ok ? HP3D_E_ARG : HP3D_E_ORDER;
         return;
     }
-    sf_fill_tab<WGS>(es, tb, tid);
+    sf_fill_tab<WGS>(es.m, tb, tid);
     sf_fill_rows<SPACE>(es, row, tid, WGS);
     if (a.ngeo != 8) sf_fill_gmap(es, a.ngeo, gmap, tid, WGS);
     lds_barrier();
@@ -1156,7 +1168,7 @@ __global__ __launch_bounds__(WGS, WPE) void sf_elem_kernel(ElemArgs a)
     lds_barrier();
     if (part == nparts - 1 && a.bout) {
         double *bo = a.bout + a.off_v[e];
-        sf_load<SPACE, WGS>(es, tb, row, pool, [=](int r, double v) { bo[r] = v; }, tid);
+        sf_load<SPACE, WGS>(es, tb, row, pool + (SPACE == 0 ? 6 : 12) * es.nint, [=](int r, double v) { bo[r] = v; }, tid);
     }
     const SfToK<T> to{(T *)a.kout + a.off_k[e], a.ld_k > 0 ? a.ld_k : es.n};
     const int dl = (sf_fields(SPACE) * es.nint + 1) & ~1;
@@ -1609,7 +1621,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void sf_fused_kernel(SingleArgs sa)
             continue;
         }
         if (tid == 0) sm.fail = 0;
-        sf_fill_tab<WGS>(es, tb, tid);
+        sf_fill_tab<WGS>(es.m, tb, tid);
         sf_fill_rows<SPACE>(es, row, tid, WGS);
         if (a.ngeo != 8) sf_fill_gmap(es, a.ngeo, gmap, tid, WGS);
         lds_barrier();
@@ -1621,7 +1633,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void sf_fused_kernel(SingleArgs sa)
         lds_barrier();
         {
             double *const bl = sm.b, *const bo = a.bout ? a.bout + a.off_v[e] : nullptr;
-            sf_load<SPACE, WGS>(es, tb, row, d,
+            sf_load<SPACE, WGS>(es, tb, row, d + (SPACE == 0 ? 6 : 12) * es.nint,
                                 [=](int r, double v) {
                                     bl[r] = v;
                                     if (bo) bo[r] = v;
@@ -1667,4 +1679,332 @@ __global__ __launch_bounds__(64 * NW, WPE) void sf_fused_kernel(SingleArgs sa)
         sf_condense<T, NBT, R, NW, true>(a, cd, e, es, pool, pool + ly.kb, ly, NBT > 1 ? wbuf : pool + ly.len, sm, tid);
     }
 #endif
+}
+
+// ------------------------------------------------------- field evaluation
+//
+// One workgroup per element evaluates finite-element fields from element dof
+// vectors at the quadrature points (soleval, element/util/soleval.F90, with
+// the dofs in element order) and integrates one of:
+//   HP3D_FIELD_ERROR    element_error (element/util/compute_error.F90:226-400):
+//                       set_3Dint rule with INTEGRATION = 2; out[2e] = errorH
+//                       (int |grad(u - u_h)|^2 + |u - u_h|^2) or errorE (curl
+//                       and value), out[2e+1] = the same norm of the exact u
+//   HP3D_FIELD_ADJOINT  out[e] = -coef_e int grad v_h . grad u_h (H1) or
+//                       -coef_e int v_h . u_h (H(curl)): lambda_e^T (dK_e /
+//                       dlog coef_e) u_e with a minus sign, i.e. dJ/dtheta_e
+//                       for coef = exp(theta), recomputed at the points of the
+//                       element rule without forming K_e
+//   HP3D_FIELD_L2       out[e] = int u_h . u_h and r[off_v[e] + k] = int
+//                       phi_k . u_h (the element mass matrix times u_e)
+// The dofs are summed one direction after the other (C, B, then A at the
+// point), value and reference derivatives at once, and r goes the same way
+// back: O(m^4) work where a sum over all dofs at every point is O(m^6).  What
+// is left is mostly the points themselves (map, exact solution).  On 13,824
+// H1 p = 3 elements (216 points, ERROR) 0.490 -> 0.117 ms, on 4,080 p = 4
+// elements ADJOINT and L2 0.263 -> 0.040 ms each.
+struct FieldArgs {
+    int space, mode, nel, ngeo, exact;
+    const int *norder, *nori_e, *nori_f;
+    const double *xnod, *coef;
+    const long long *off_v;
+    const double *u, *v;
+    double *out, *r;
+    int *status;
+};
+
+// exact solutions of the manufactured problems (value, gradient); the
+// selector is the load selector of the same problem
+__device__ inline void exact_h1(int sel, const double *x, double &u, double *du)
+{
+    const double pi = 3.14159265358979323846;
+    u = du[0] = du[1] = du[2] = 0.0;
+    if (sel == HP3D_LOAD_SINSINSIN) {
+        double s[3], c[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) sincospi(x[i], &s[i], &c[i]);
+        u = s[0] * s[1] * s[2];
+        du[0] = pi * c[0] * s[1] * s[2];
+        du[1] = pi * s[0] * c[1] * s[2];
+        du[2] = pi * s[0] * s[1] * c[2];
+    } else if (sel == HP3D_LOAD_CONV) {
+        double sx, cx;
+        sincospi(x[0], &sx, &cx);
+        const double sh = sinh(pi * x[1]), z2 = x[2] * x[2];
+        u = sx * sh * z2;
+        du[0] = pi * cx * sh * z2;
+        du[1] = pi * sx * cosh(pi * x[1]) * z2;
+        du[2] = 2.0 * sx * sh * x[2];
+    } else if (sel == HP3D_LOAD_POLY2) {
+        double a0 = x[0] * (1.0 - x[0]), a1 = x[1] * (1.0 - x[1]), a2 = x[2] * (1.0 - x[2]);
+        u = a0 * a1 * a2;
+        du[0] = (1.0 - 2.0 * x[0]) * a1 * a2;
+        du[1] = a0 * (1.0 - 2.0 * x[1]) * a2;
+        du[2] = a0 * a1 * (1.0 - 2.0 * x[2]);
+    } else if (sel == HP3D_LOAD_XYZ) {
+        u = x[0] * x[1] * x[2];
+        du[0] = x[1] * x[2];
+        du[1] = x[0] * x[2];
+        du[2] = x[0] * x[1];
+    }
+}
+
+__device__ inline void exact_hcurl(int sel, const double *x, double *e, double *curl)
+{
+    const double pi = 3.14159265358979323846;
+    for (int i = 0; i < 3; ++i) e[i] = curl[i] = 0.0;
+    if (sel == HP3D_LOAD_CURL_SIN) {
+        double sy, cy, sz, cz;
+        sincospi(x[1], &sy, &cy);
+        sincospi(x[2], &sz, &cz);
+        e[0] = sy * sz;
+        curl[1] = pi * sy * cz;
+        curl[2] = -pi * cy * sz;
+    }
+}
+
+// points per direction (by role) of the set_3Dint brick rule with INTEGRATION
+// = 2 (set_3D_int.F90:8-21,203-244): face orders as coded (no swap), orders
+// raised by 2 and capped at MAXP; direction d by the calling lane
+__device__ __forceinline__ int sf_rule_plain(const SfElem &es, int d)
+{
+    int m = es.o.b[d];
+    for (int i = 0; i < 4; ++i) m = max(m, es.o.pe[d == 2 ? 8 + i : 2 * i + d]);
+    // faces 0..5 have axes (0,1), (0,1), (0,2), (1,2), (0,2), (1,2)
+    const int h = d == 0 ? 0x17 : d == 1 ? 0x28 : 0, v = d == 1 ? 0x03 : d == 2 ? 0x3c : 0;
+    for (int f = 0; f < 6; ++f) {
+        if (h >> f & 1) m = max(m, es.o.fh[f]);
+        if (v >> f & 1) m = max(m, es.o.fv[f]);
+    }
+    return min(m + 2, MAXP) + 1;
+}
+
+// u_h's dofs summed over C, then B: y[3 (comp (mA nB nC) + (iA nB + qB) nC + qC) ..]
+// = the value chain, the one with the derivative in B, the one in C; c may be y
+template <int SPACE, int WGS>
+__device__ __forceinline__ void sf_field_sums(const SfElem &es, const SfTab &tb, const int (&nq)[3], const short *row,
+                                              const double *u, double *c, double *x, double *y, int tid)
+{
+    constexpr int NC = sf_comps(SPACE), DER = SF_I * 8;
+    const int mA = es.m[1], mB = es.m[0], mC = es.m[2], nB = nq[0], nC = nq[2];
+    for (int k = tid; k < NC * mA * mB * mC; k += WGS) {
+        const int k1 = k / mC, iC = k - k1 * mC, k2 = k1 / mB, iB = k1 - k2 * mB, a = k2 / mA, iA = k2 - a * mA;
+        const int r = row[((a * SF_I + iA) * SF_I + iB) * 8 + iC];
+        const double v = r < 0 ? 0.0 : u[r & ~ROW_NEG];
+        c[k] = r & ROW_NEG ? -v : v;
+    }
+    lds_barrier();
+    for (int k = tid; k < NC * mA * mB * nC; k += WGS) {
+        const int k1 = k / nC, qC = k - k1 * nC, a = SPACE == 0 ? -1 : k1 / (mA * mB);
+        const double *f = tb.f[2][0] + qC, *ck = c + k1 * mC;
+        const int v = a == 2 ? DER : 0;
+        double s0 = 0.0, s1 = 0.0;
+        for (int i = 0; i < mC; ++i) {
+            s0 = fma(f[v + 8 * i], ck[i], s0);
+            s1 = fma(f[DER + 8 * i], ck[i], s1);
+        }
+        x[2 * k] = s0;
+        x[2 * k + 1] = s1;
+    }
+    lds_barrier();
+    for (int k = tid; k < NC * mA * nB * nC; k += WGS) {
+        const int k1 = k / nC, qC = k - k1 * nC, k2 = k1 / nB, qB = k1 - k2 * nB, a = SPACE == 0 ? -1 : k2 / mA;
+        const double *f = tb.f[0][0] + qB, *xk = x + 2 * (k2 * mB * nC + qC);
+        const int v = a == 0 ? DER : 0;
+        double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+        for (int i = 0; i < mB; ++i) {
+            const double x0 = xk[2 * i * nC], x1 = xk[2 * i * nC + 1];
+            s0 = fma(f[v + 8 * i], x0, s0);
+            s1 = fma(f[DER + 8 * i], x0, s1);
+            s2 = fma(f[v + 8 * i], x1, s2);
+        }
+        y[3 * k] = s0;
+        y[3 * k + 1] = s1;
+        y[3 * k + 2] = s2;
+    }
+    lds_barrier();
+}
+
+// the field in reference form at point (qA, qB, qC): value and gradient (H1)
+// or E and curl E (H(curl))
+template <int SPACE>
+__device__ __forceinline__ void sf_field_at(const SfElem &es, const SfTab &tb, const int (&nq)[3], const double *y, int qA,
+                                            int qB, int qC, double (&f)[3], double (&g)[3])
+{
+    constexpr int DER = SF_I * 8;
+    const int mA = es.m[1], nB = nq[0], nC = nq[2];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) f[j] = g[j] = 0.0;
+#pragma unroll
+    for (int a = 0; a < sf_comps(SPACE); ++a) { // (the roles B, A, C are x, y, z)
+        const double *t = tb.f[1][0] + qA, *ya = y + 3 * ((a * mA * nB + qB) * nC + qC);
+        const int v = SPACE == 1 && a == 1 ? DER : 0;
+        double s = 0.0, dx = 0.0, dy = 0.0, dz = 0.0;
+        for (int i = 0; i < mA; ++i, ya += 3 * nB * nC) {
+            const double y0 = ya[0], fa = t[v + 8 * i];
+            s = fma(fa, y0, s);
+            dy = fma(t[DER + 8 * i], y0, dy);
+            dx = fma(fa, ya[1], dx);
+            dz = fma(fa, ya[2], dz);
+        }
+        if (SPACE == 0) {
+            f[0] = s;
+            g[0] = dx;
+            g[1] = dy;
+            g[2] = dz;
+        } else { // curl (s e_a) = grad s x e_a
+            f[a] = s;
+            if (a == 0) {
+                g[1] += dz;
+                g[2] -= dy;
+            } else if (a == 1) {
+                g[0] -= dz;
+                g[2] += dx;
+            } else {
+                g[0] += dy;
+                g[1] -= dx;
+            }
+        }
+    }
+}
+
+// covariant transform: gradients of H1, values of H(curl)
+__device__ __forceinline__ void sf_covariant(const double (&inv)[3][3], const double (&g)[3], double (&out)[3])
+{
+#pragma unroll
+    for (int j = 0; j < 3; ++j) out[j] = g[0] * inv[0][j] + g[1] * inv[1][j] + g[2] * inv[2][j];
+}
+
+// PAIR: ADJOINT (two fields); otherwise ERROR or L2
+template <int SPACE, bool PAIR>
+__global__ __launch_bounds__(128, SPACE == 0 ? 3 : 2) void field_kernel(FieldArgs fa)
+{
+    constexpr int WGS = 128, NU = (MAXQ + WGS - 1) / WGS, NC = sf_comps(SPACE);
+    __shared__ SfElem es;
+    __shared__ SfTab tb;
+    __shared__ __align__(16) short row[NC * SF_I * SF_I * 8];
+    __shared__ double xg[SF_XG];
+    __shared__ double x[2 * NC * MAXQ], y[3 * NC * MAXQ];
+    __shared__ double red[2][WGS / 64];
+    __shared__ int rule[3];
+    unsigned short *const gmap = reinterpret_cast<unsigned short *>(xg + 3 * XS_MAX + 1);
+    const int e = blockIdx.x, tid = threadIdx.x;
+    ElemArgs a;
+    a.ngeo = fa.ngeo;
+    a.norder = fa.norder;
+    a.nori_e = fa.nori_e;
+    a.nori_f = fa.nori_f;
+    a.xnod = fa.xnod;
+    a.coef = fa.coef;
+    if (!sf_setup<SPACE, WGS>(a, e, es, xg, tid)) {
+        if (tid == 0 && fa.status) fa.status[e] = HP3D_E_ORDER;
+        return;
+    }
+    const bool err = !PAIR && fa.mode == HP3D_FIELD_ERROR;
+    if (tid < 3) rule[tid] = err ? sf_rule_plain(es, tid) : es.m[tid];
+    sf_fill_rows<SPACE>(es, row, tid, WGS);
+    if (fa.ngeo != 8) sf_fill_gmap(es, fa.ngeo, gmap, tid, WGS);
+    lds_barrier();
+    const int nq[3] = {rule[0], rule[1], rule[2]}, Q = nq[0] * nq[1] * nq[2];
+    sf_fill_tab<WGS>(nq, tb, tid);
+    lds_barrier();
+    // of the pair, v's part (reference gradient or value) waits in registers
+    double hv[PAIR ? NU : 1][3];
+    if constexpr (PAIR) {
+        sf_field_sums<SPACE, WGS>(es, tb, nq, row, fa.v + fa.off_v[e], y, x, y, tid);
+#pragma unroll
+        for (int i = 0; i < NU; ++i) {
+            const int l = min(tid + i * WGS, Q - 1), l1 = l / nq[2], qC = l - l1 * nq[2], qA = l1 / nq[0];
+            double f[3], g[3];
+            sf_field_at<SPACE>(es, tb, nq, y, qA, l1 - qA * nq[0], qC, f, g);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) hv[i][j] = SPACE == 0 ? g[j] : f[j];
+        }
+        lds_barrier();
+    }
+    sf_field_sums<SPACE, WGS>(es, tb, nq, row, fa.u + fa.off_v[e], y, x, y, tid);
+
+    const bool staged = fa.ngeo <= XS_MAX;
+    const double coef = xg[3 * XS_MAX];
+    double acc0 = 0.0, acc1 = 0.0;
+    bool neg = false;
+    double *const pw = x; // weighted field of L2
+    auto point = [&](int l, const double (&h)[3]) __attribute__((always_inline)) {
+        const int l1 = l / nq[2], qC = l - l1 * nq[2], qA = l1 / nq[0], qB = l1 - qA * nq[0];
+        double f[3], g[3], xp[3], jm[3][3], inv[3][3], t[3];
+        sf_field_at<SPACE>(es, tb, nq, y, qA, qB, qC, f, g);
+        const double det = staged ? sf_map<true>(es, tb, gmap, xg, fa.ngeo, qB, qA, qC, xp, jm, inv)
+                                  : sf_map<false>(es, tb, gmap, fa.xnod + 3 * (size_t)fa.ngeo * e, fa.ngeo, qB, qA, qC,
+                                                  xp, jm, inv);
+        neg = neg || det < 0.0;
+        const double wd = det * (tb.w[0][qB] * tb.w[1][qA] * tb.w[2][qC]);
+        sf_covariant(inv, SPACE == 0 ? g : f, t);
+        if constexpr (PAIR) {
+            double tv[3];
+            sf_covariant(inv, h, tv);
+            acc0 -= coef * (t[0] * tv[0] + t[1] * tv[1] + t[2] * tv[2]) * wd;
+        } else if (err) {
+            double fe[3], ge[3], fu[3], gu[3];
+            if (SPACE == 0) {
+                exact_h1(fa.exact, xp, fe[0], ge);
+                fe[1] = fe[2] = fu[1] = fu[2] = 0.0;
+                fu[0] = f[0];
+            } else {
+                exact_hcurl(fa.exact, xp, fe, ge);
+            }
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                if (SPACE == 0) {
+                    gu[j] = t[j];
+                } else {
+                    fu[j] = t[j];
+                    gu[j] = (jm[j][0] * g[0] + jm[j][1] * g[1] + jm[j][2] * g[2]) / det;
+                }
+                acc0 += ((ge[j] - gu[j]) * (ge[j] - gu[j]) + (fe[j] - fu[j]) * (fe[j] - fu[j])) * wd;
+                acc1 += (ge[j] * ge[j] + fe[j] * fe[j]) * wd;
+            }
+        } else {
+            // weighted field pulled back to reference components: phi_k . u_h w det
+            if (SPACE == 0) {
+                acc0 += f[0] * f[0] * wd;
+                pw[l] = f[0] * wd;
+            } else {
+                acc0 += (t[0] * t[0] + t[1] * t[1] + t[2] * t[2]) * wd;
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                    pw[i * Q + l] = (inv[i][0] * t[0] + inv[i][1] * t[1] + inv[i][2] * t[2]) * wd;
+            }
+        }
+    };
+    if constexpr (PAIR) {
+#pragma unroll
+        for (int i = 0; i < NU; ++i)
+            if (tid + i * WGS < Q) point(tid + i * WGS, hv[i]);
+    } else {
+        for (int l = tid; l < Q; l += WGS) point(l, hv[0]);
+    }
+    if (neg) es.negjac = 1;
+    // workgroup sums
+    for (int off = 32; off > 0; off >>= 1) {
+        acc0 += __shfl_down(acc0, off);
+        acc1 += __shfl_down(acc1, off);
+    }
+    if ((tid & 63) == 0) {
+        red[0][tid >> 6] = acc0;
+        red[1][tid >> 6] = acc1;
+    }
+    lds_barrier();
+    if (tid == 0) {
+        if (err) {
+            fa.out[2 * (size_t)e] = red[0][0] + red[0][1];
+            fa.out[2 * (size_t)e + 1] = red[1][0] + red[1][1];
+        } else {
+            fa.out[e] = red[0][0] + red[0][1];
+        }
+        if (fa.status) fa.status[e] = es.negjac ? HP3D_NEG_JACOBIAN : 0;
+    }
+    if (!PAIR && fa.mode == HP3D_FIELD_L2 && fa.r) {
+        double *re = fa.r + fa.off_v[e];
+        sf_load<SPACE, WGS>(es, tb, row, pw, [=](int k, double v) { re[k] = v; }, tid);
+    }
 }

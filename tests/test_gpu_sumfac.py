@@ -137,3 +137,48 @@ def test_fused_anisotropic(gpu, space, porder):
     m = mesh.structured((2, 1, 1), porder=porder, perm_seed=5 + sum(porder), coef=[0.7, 1.9])
     x = m.xnod() + 0.05 * np.random.default_rng(sum(porder)).uniform(-1, 1, (2, 8, 3))
     condensed_against_oracle(space, m.norder, m.nori_e, m.nori_f, x, m.coef, FUSED)
+
+
+@pytest.mark.parametrize("space", [0, 1])
+@pytest.mark.parametrize("ngeo", [8, 27, 343])
+def test_field_any_codes(gpu, space, ngeo):
+    """The field integrals at any orders and orientations (ngeo = 8) and with
+    isoparametric maps, staged (27 nodes) and not (343).  Tolerance: the field
+    at a point sums up to 343 products of O(1) dofs, 343 eps < 1e-13 of the
+    field's own size; the integrals are quadratic in it and their weights carry
+    a few eps more, so 1e-12 of their norms."""
+    import torch
+
+    import hp3d_amd
+    from hp3d_amd import FIELD_ADJOINT, FIELD_ERROR, FIELD_L2
+    from hp3d_amd.solve import field
+
+    rng = np.random.default_rng(90 + space + ngeo)
+    nel = 24 if ngeo == 8 else 4
+    no, oe, of = random_codes(rng, nel, 6)
+    if ngeo > 8:
+        p = 2 if ngeo == 27 else 6
+        no[:, :12], no[:, 12:18], no[:, 18] = p, 11 * p, 111 * p
+    x = np.zeros((nel, ngeo, 3))
+    x[:, :8] = mesh.VERT_XYZ[None] + 0.15 * rng.uniform(-1, 1, (nel, 8, 3))
+    x[:, 8:] = 0.2 / ngeo * rng.uniform(-1, 1, (nel, ngeo - 8, 3))
+    coef = rng.uniform(0.5, 2.0, nel)
+    sel = oracle.LOAD_SINSINSIN if space == 0 else oracle.LOAD_CURL_SIN
+    batch = hp3d_amd.ElementBatch(space, no, oe, of, x, coef, load=sel)
+    u = torch.as_tensor(rng.normal(size=batch.size_v), device="cuda")
+    v = torch.as_tensor(rng.normal(size=batch.size_v), device="cuda")
+    err = field(batch, FIELD_ERROR, u, exact=sel)[0].cpu().numpy()
+    l2, r = field(batch, FIELD_L2, u, with_r=True)
+    adj = field(batch, FIELD_ADJOINT, u, v=v)[0].cpu().numpy()
+    assert (batch.check_status() == 0).all()
+    l2 = l2.cpu().numpy()
+    for e in range(nel):
+        i = int(batch.iperm[e])
+        o, n = int(batch.off_v_h[i]), int(batch._n[i])
+        ue, ve, re = (t[o:o + n].cpu().numpy() for t in (u, v, r))
+        assert rel(err[i], np.array(oracle.element_error(space, no[e], oe[e], of[e], x[e].T, ue, sel))) < 1e-12, e
+        mm = oracle.elem_mass(space, no[e], oe[e], of[e], x[e].T)
+        assert abs(l2[i] - ue @ mm @ ue) < 1e-12 * (ue @ mm @ ue), e
+        assert rel(re, mm @ ue) < 1e-12, e
+        k = oracle.elem_h1(no[e], oe[e], of[e], x[e].T, kappa=coef[e])[0] if space == 0 else coef[e] * mm
+        assert abs(adj[i] + ve @ k @ ue) < 1e-12 * np.sqrt((ve @ k @ ve) * (ue @ k @ ue)), e
