@@ -2169,22 +2169,98 @@ struct BwdArgs {
     double *x;
 };
 
+// Interface and bubble counts of one element by a whole wave (lane l: header
+// integer l); false (uniformly) for invalid orders.
+__device__ __forceinline__ bool wave_counts(int space, const int *norder, int lane, int &ni, int &nb)
+{
+    const int v = lane < 19 ? norder[lane] : 1;
+    bool ok = true;
+    int c = 0;
+    if (lane < 12) {
+        ok = v >= 1 && v <= MAXP;
+        c = space == HP3D_H1 ? v - 1 : v;
+    } else if (lane < 18) {
+        const int h = v / MODORDER, w = v % MODORDER;
+        ok = h >= 1 && h <= MAXP && w >= 1 && w <= MAXP;
+        c = space == HP3D_H1 ? (h - 1) * (w - 1) : h * (w - 1) + (h - 1) * w;
+    } else if (lane == 18) {
+        const int x = v / 100, y = (v / 10) % 10, z = v % 10;
+        ok = x >= 1 && x <= MAXP && y >= 1 && y <= MAXP && z >= 1 && z <= MAXP;
+        c = space == HP3D_H1 ? (x - 1) * (y - 1) * (z - 1)
+                             : x * (y - 1) * (z - 1) + (x - 1) * y * (z - 1) + (x - 1) * (y - 1) * z;
+    }
+    nb = __builtin_amdgcn_readlane(c, 18);
+    const int sum = sf_scan(lane < 18 ? c : 0, [](int x, int y) { return x + y; });
+    ni = __builtin_amdgcn_readlane(sum, 31) + (space == HP3D_H1 ? 8 : 0);
+    return __all(ok);
+}
+
+// Sum over i in [lo, hi) of A[i nb + q0 + q] x[i] for the w <= 64 columns at
+// q0, in lanes q < w: the lanes split into 64 / w groups of w, so that a step
+// reads consecutive rows in one piece.
+__device__ __forceinline__ double wave_columns(const double *A, const double *x, int nb, int lo, int hi, int q0, int w,
+                                               int lane)
+{
+    constexpr int U = 8;
+    const int groups = 64 / w, g = lane / w, q = lane - g * w;
+    double s = 0.0;
+    if (g < groups)
+        for (int i0 = lo + g; i0 < hi; i0 += U * groups) {
+            double av[U], xv[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int i = min(i0 + u * groups, hi - 1);
+                av[u] = A[(size_t)i * nb + q0 + q];
+                xv[u] = x[i];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (i0 + u * groups < hi) s = fma(av[u], xv[u], s);
+        }
+    for (int c = groups; c > 1;) { // tree over the groups
+        const int h = (c + 1) >> 1;
+        const double t = __shfl(s, lane + h * w);
+        if (g + h < c) s += t;
+        c = h;
+    }
+    return s;
+}
+
+// One wave per element, or one workgroup (NE = 1: each wave sums a quarter of
+// the interface) where the elements are too few to fill the chip.  Bound by
+// reading ASchur: with one thread per bubble and every thread decoding the
+// orders by itself 13,824 H1 p = 3 elements (50 MB) took 74 us, now 14; 4,096
+// p = 4 elements 42 -> 19, 512 H(curl) p = 6 elements (0.8 GB) 398 -> 175.
+// BWD_WAVES: one wave for each SIMD of the chip.  A workgroup each is the
+// better one below (64 H1 p = 6 elements 11 us, waves 28; 1,000 of H(curl)
+// p = 5 137 and 145), waves above (13,824 p = 3 elements 14 us, workgroups 37).
+constexpr int BWD_WAVES = 1024;
+template <int NE>
 __global__ __launch_bounds__(WG) void stc_bwd_kernel(BwdArgs a)
 {
-    const int e = blockIdx.x;
-    const int *no = a.norder + 19 * (size_t)e;
-    int zero[18] = {0};
-    ElemOrders o;
-    if (!decode_orders(no, zero, zero + 12, o)) return;
-    int n, nb;
-    dof_counts(a.space, o, n, nb);
-    int ni = n - nb;
-    const double *A = a.aschur + a.off_s[e];
+    constexpr int NW = WG / 64;
+    static_assert(NE == 1 || NE == NW, "elements per workgroup");
+    __shared__ double part[NE == 1 ? NW : 1][NE == 1 ? MAXN_E / 2 + 64 : 1];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int e = NE == 1 ? blockIdx.x : blockIdx.x * NE + wave;
+    if (e >= a.nel) return;
+    int ni, nb;
+    if (!wave_counts(a.space, a.norder + 19 * (size_t)e, lane, ni, nb)) return;
+    const double *A = a.aschur + a.off_s[e], *bs = a.bschur + a.off_v[e];
     double *x = a.x + a.off_v[e];
-    for (int q = threadIdx.x; q < nb; q += WG) {
-        double s = 0.0;
-        for (int i = 0; i < ni; ++i) s += A[(size_t)i * nb + q] * x[i];
-        x[ni + q] = a.bschur[a.off_v[e] + q] - s;
+    const int lo = NE == 1 ? ni * wave / NW : 0, hi = NE == 1 ? ni * (wave + 1) / NW : ni;
+    for (int q0 = 0; q0 < nb; q0 += 64) {
+        const int w = min(64, nb - q0);
+        const double s = wave_columns(A, x, nb, lo, hi, q0, w, lane);
+        if (lane < w) {
+            if (NE == 1) part[wave][q0 + lane] = s;
+            else x[ni + q0 + lane] = bs[q0 + lane] - s;
+        }
+    }
+    if constexpr (NE == 1) {
+        __syncthreads();
+        for (int q = threadIdx.x; q < nb; q += WG)
+            x[ni + q] = bs[q] - ((part[0][q] + part[1][q]) + (part[2][q] + part[3][q]));
     }
 }
 
@@ -2225,33 +2301,67 @@ __global__ __launch_bounds__(WG) void dirichlet_lift_kernel(LiftArgs a)
 // matrices (vectors), this is the assembly of the element systems into CSR
 // values (mumps_sc.F90:266-323 accumulates the same triplets, duplicates
 // summed); the fixed summation order makes it deterministic.
-__global__ __launch_bounds__(WG) void gather_sum_kernel(long long nout, const long long *ptr,
-                                                       const long long *src, const double *in,
-                                                       double *out)
+// Bound by the lines of in: consecutive outputs are a row of the global matrix
+// and lie a column of Aii apart, so each of them reads 8 bytes of a line that
+// the next rows of the node read again.  Rows that follow one another
+// therefore go to one XCD, whose L2 keeps the lines: 29.4M values of 13,824 H1
+// p = 3 elements 0.528 -> 0.420 ms, 26.8M of 4,096 p = 4 elements 0.51 -> 0.35.
+// (Runs of 16 or 64 workgroups are alike; one contiguous eighth per XCD is
+// slower, 0.67 ms, the rows of vertices, edges and faces being unequal; so are
+// two or four outputs per thread, 0.43 and 0.465.)
+constexpr int GATHER_WG = 256;
+constexpr unsigned XCDS = 8, XCD_RUN = 16;
+// the part of the work that workgroup b of n takes: workgroups go round the
+// XCDs in turn, and of XCDS * XCD_RUN parts an XCD takes XCD_RUN that follow
+// one another
+__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned n)
 {
-    long long t = (long long)blockIdx.x * WG + threadIdx.x;
+    const unsigned i = b % (XCDS * XCD_RUN), b0 = b - i;
+    return b0 + XCDS * XCD_RUN <= n ? b0 + i % XCDS * XCD_RUN + i / XCDS : b;
+}
+__global__ __launch_bounds__(GATHER_WG) void gather_sum_kernel(long long nout, const long long *ptr,
+                                                              const long long *src, const double *in,
+                                                              double *out)
+{
+    const long long t = (long long)xcd_block(blockIdx.x, gridDim.x) * GATHER_WG + threadIdx.x;
     if (t >= nout) return;
     double s = 0.0;
     for (long long j = ptr[t]; j < ptr[t + 1]; ++j) s += in[src[j]];
     out[t] = s;
 }
 
-// y = A x for a CSR matrix (FP64 values, int32 column indices): 32 lanes per
-// row, each lane striding over the row's nonzeros (coalesced reads of
-// indices and values), then a 32-lane shuffle reduction.  HBM bound: 12
-// bytes per nonzero plus the gathered x.  The global condensed systems have
-// tens to hundreds of nonzeros per row.
-constexpr int SPMV_LPR = 32;
+// y = A x for a CSR matrix (FP64 values, int32 column indices): 16 lanes per
+// row, each lane striding over the row's nonzeros, four of them in flight, then
+// a shuffle reduction.  HBM bound: 12 bytes per nonzero plus the gathered x
+// (29.4M nonzeros 0.101 -> 0.089 ms, 4.0 TB/s; 26.8M in rows of 190 0.083 ->
+// 0.067; 32 lanes with four in flight 0.096, 64 lanes 0.122).  The global
+// condensed systems have tens to hundreds of nonzeros per row.
+constexpr int SPMV_LPR = 16;
 __global__ __launch_bounds__(WG) void csr_spmv_kernel(long long nrows, const long long *indptr,
                                                      const int *indices, const double *vals,
                                                      const double *x, double *y)
 {
-    long long row = (long long)blockIdx.x * (WG / SPMV_LPR) + threadIdx.x / SPMV_LPR;
+    constexpr int U = 4;
+    const long long row = (long long)blockIdx.x * (WG / SPMV_LPR) + threadIdx.x / SPMV_LPR;
     const int sub = threadIdx.x % SPMV_LPR;
     double s = 0.0;
     if (row < nrows) {
-        for (long long j = indptr[row] + sub; j < indptr[row + 1]; j += SPMV_LPR)
-            s += vals[j] * x[indices[j]];
+        const long long end = indptr[row + 1];
+        for (long long j0 = indptr[row] + sub; j0 < end; j0 += U * SPMV_LPR) {
+            double v[U], xv[U];
+            int c[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const long long j = min(j0 + u * SPMV_LPR, end - 1);
+                v[u] = vals[j];
+                c[u] = indices[j];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) xv[u] = x[c[u]];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (j0 + u * SPMV_LPR < end) s += v[u] * xv[u];
+        }
     }
     for (int off = SPMV_LPR / 2; off > 0; off >>= 1) s += __shfl_down(s, off, SPMV_LPR);
     if (row < nrows && sub == 0) y[row] = s;
@@ -2790,7 +2900,8 @@ int hp3d_gpu_stc_bwd_batch(int space, int nel, const int *norder, const long lon
     if (nel == 0) return 0;
     if (!norder || !off_s || !aschur || !off_v || !bschur || !x) return HP3D_E_ARG;
     BwdArgs a{space, nel, norder, off_s, off_v, aschur, bschur, x};
-    hipLaunchKernelGGL(stc_bwd_kernel, dim3(nel), dim3(WG), 0, (hipStream_t)stream, a);
+    if (nel >= BWD_WAVES) hipLaunchKernelGGL(stc_bwd_kernel<WG / 64>, dim3((nel + WG / 64 - 1) / (WG / 64)), dim3(WG), 0, (hipStream_t)stream, a);
+    else hipLaunchKernelGGL(stc_bwd_kernel<1>, dim3(nel), dim3(WG), 0, (hipStream_t)stream, a);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -2878,7 +2989,8 @@ int hp3d_gpu_gather_sum(long long nout, const long long *ptr, const long long *s
     if (!ptr || !src || !in || !out) return HP3D_E_ARG;
     long long nblk = (nout + WG - 1) / WG;
     if (nblk > 0x7fffffffLL) return HP3D_E_ARG;
-    hipLaunchKernelGGL(gather_sum_kernel, dim3((unsigned)nblk), dim3(WG), 0, (hipStream_t)stream,
+    nblk = (nout + GATHER_WG - 1) / GATHER_WG;
+    hipLaunchKernelGGL(gather_sum_kernel, dim3((unsigned)nblk), dim3(GATHER_WG), 0, (hipStream_t)stream,
                        nout, ptr, src, in, out);
     HIPCHK(hipGetLastError());
     return 0;
