@@ -1532,6 +1532,32 @@ struct StcArgs {
     int *status;
 };
 
+// Interface and bubble counts of one element by a whole wave (lane l: header
+// integer l); false (uniformly) for invalid orders.
+__device__ __forceinline__ bool wave_counts(int space, const int *norder, int lane, int &ni, int &nb)
+{
+    const int v = lane < 19 ? norder[lane] : 1;
+    bool ok = true;
+    int c = 0;
+    if (lane < 12) {
+        ok = v >= 1 && v <= MAXP;
+        c = space == HP3D_H1 ? v - 1 : v;
+    } else if (lane < 18) {
+        const int h = v / MODORDER, w = v % MODORDER;
+        ok = h >= 1 && h <= MAXP && w >= 1 && w <= MAXP;
+        c = space == HP3D_H1 ? (h - 1) * (w - 1) : h * (w - 1) + (h - 1) * w;
+    } else if (lane == 18) {
+        const int x = v / 100, y = (v / 10) % 10, z = v % 10;
+        ok = x >= 1 && x <= MAXP && y >= 1 && y <= MAXP && z >= 1 && z <= MAXP;
+        c = space == HP3D_H1 ? (x - 1) * (y - 1) * (z - 1)
+                             : x * (y - 1) * (z - 1) + (x - 1) * y * (z - 1) + (x - 1) * (y - 1) * z;
+    }
+    nb = __builtin_amdgcn_readlane(c, 18);
+    const int sum = sf_scan(lane < 18 ? c : 0, [](int x, int y) { return x + y; });
+    ni = __builtin_amdgcn_readlane(sum, 31) + (space == HP3D_H1 ? 8 : 0);
+    return __all(ok);
+}
+
 // ------------------------------------------------- strip condensation
 //
 // Static condensation of one element per workgroup of 8 waves, for elements
@@ -2146,9 +2172,101 @@ __global__ __launch_bounds__(64 * NW) void stc_strip_kernel(StcArgs a)
         a.status[e] = s_fail ? HP3D_E_FACTOR : (a.status[e] == HP3D_NEG_JACOBIAN ? HP3D_NEG_JACOBIAN : 0);
 }
 
+// Condensation of stored element matrices with at most R dofs and 16 NBT
+// bubbles: the upper triangle of K into LDS, then as in the fused kernel, two
+// (128 rows) or five (64 rows) workgroups a CU.  Bound by reading K's triangle
+// and writing Aii; the strips below, which go through a workspace, are built
+// for blocks of more than one MFMA tile column: 4,080 H1 p = 4 elements 1.07 ->
+// 0.23 ms.  An element whose triangle does not fit (N near 128 with 28 bubbles
+// or more) keeps only its bubble rows in LDS.
+template <typename T, int R, int NBT, int NW, int POOL, int WPE>
+__global__ __launch_bounds__(64 * NW, WPE) void stc_small_kernel(StcArgs sa)
+{
+    constexpr int WGS = 64 * NW, U = 8, H = R / 64;
+    __shared__ SfElem es;
+    __shared__ SfSmall<R> sm;
+    __shared__ double wbuf[16 * NBT * (16 * NBT + 1)]; // L^-1 of the bubble block
+    __shared__ __align__(16) double pool[POOL];
+    const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int ni, nb;
+    bool ok = true;
+    if (sa.nsz) {
+        nb = sa.nsz[2 * e + 1];
+        ni = sa.nsz[2 * e] - nb;
+    } else {
+        ok = wave_counts(sa.space, sa.norder + 19 * (size_t)e, lane, ni, nb);
+    }
+    const int n = ni + nb;
+    const int bad = !ok ? HP3D_E_ORDER
+                    : n > sa.n_max || nb > sa.nb_max ? HP3D_E_ARG
+                    : nb > 0 && ni == 0 ? HP3D_E_NOIFACE : 0;
+    if (bad) {
+        if (tid == 0 && sa.status) sa.status[e] = bad;
+        return;
+    }
+    if (tid == 0) {
+        es.n = n;
+        es.nb = nb;
+        es.negjac = sa.status && sa.status[e] == HP3D_NEG_JACOBIAN; // the warning survives
+        sm.fail = 0;
+    }
+    const T *K = (const T *)sa.kin + sa.off_k[e];
+    const size_t ldk = sa.ld_k > 0 ? (size_t)sa.ld_k : (size_t)n, ldc = sa.ld_c > 0 ? (size_t)sa.ld_c : (size_t)ni;
+    const double *b = sa.bin + sa.off_v[e];
+    double *const aii = sa.aii + sa.off_c[e];
+    const SfLay ly(n, nb, 16 * NBT);
+    const bool packed = ly.len <= POOL;
+    // column c of K's upper triangle is row c of SfLay's; without room for all
+    // of them the interface block goes to (or, condensed in place, is in)
+    // Aii's memory, and the bubble rows start the pool
+    double *const kb = packed ? pool + ly.kb : pool;
+    for (int c = (packed ? 0 : ni) + wv; c < n; c += NW * U) {
+        T v[U][H];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const T *col = K + min(c + u * NW, n - 1) * ldk;
+#pragma unroll
+            for (int h = 0; h < H; ++h) v[u][h] = col[min(lane + 64 * h, n - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int cu = c + u * NW;
+            if (cu >= n) break;
+            double *o = cu < ni ? pool + ly.row(cu) : kb + (cu - ni) * ly.ldb;
+#pragma unroll
+            for (int h = 0; h < H; ++h)
+                if (lane + 64 * h <= cu) o[lane + 64 * h] = (double)v[u][h];
+        }
+    }
+    if (!packed && (const void *)aii != (const void *)K)
+        for (int k = tid; k < ni * ni; k += WGS) {
+            const int c = k / ni, r = k - c * ni;
+            if (c <= r) aii[r + c * ldc] = (double)K[c + r * ldk];
+        }
+    for (int k = tid; k < n; k += WGS) sm.b[k] = b[k];
+    __syncthreads();
+    ElemArgs a;
+    a.kout = nullptr;
+    a.off_v = sa.off_v;
+    a.status = sa.status;
+    const CondArgs cd{sa.off_c, sa.off_s, sa.aii, sa.bi, sa.aschur, sa.bschur};
+    if (packed) sf_condense<T, NBT, R, NW, true>(a, cd, e, es, pool, kb, ly, wbuf, sm, ldc, tid);
+    else sf_condense<T, NBT, R, NW, false>(a, cd, e, es, nullptr, kb, ly, wbuf, sm, ldc, tid);
+}
+
 template <typename T>
 static void launch_stc(StcArgs a, int max_nbubble, hipStream_t st)
 {
+    // elements that one workgroup's LDS holds (4,080 of 98 + 27 dofs 0.23 ms,
+    // by strips 1.07)
+    if (a.n_max <= BR / 2 && max_nbubble <= NBF / 2) {
+        hipLaunchKernelGGL((stc_small_kernel<T, 64, 1, 4, 3264, 4>), dim3(a.nel), dim3(256), 0, st, a);
+        return;
+    }
+    if (a.n_max <= BR && max_nbubble <= NBF) {
+        hipLaunchKernelGGL((stc_small_kernel<T, 128, 2, 8, 8352, 4>), dim3(a.nel), dim3(512), 0, st, a);
+        return;
+    }
     // 64-column strips (2 block rows per wave) up to 256 bubbles, with the
     // register-resident Cholesky up to 240; 32-column strips (4 block rows
     // per wave) beyond
@@ -2168,32 +2286,6 @@ struct BwdArgs {
     const double *aschur, *bschur;
     double *x;
 };
-
-// Interface and bubble counts of one element by a whole wave (lane l: header
-// integer l); false (uniformly) for invalid orders.
-__device__ __forceinline__ bool wave_counts(int space, const int *norder, int lane, int &ni, int &nb)
-{
-    const int v = lane < 19 ? norder[lane] : 1;
-    bool ok = true;
-    int c = 0;
-    if (lane < 12) {
-        ok = v >= 1 && v <= MAXP;
-        c = space == HP3D_H1 ? v - 1 : v;
-    } else if (lane < 18) {
-        const int h = v / MODORDER, w = v % MODORDER;
-        ok = h >= 1 && h <= MAXP && w >= 1 && w <= MAXP;
-        c = space == HP3D_H1 ? (h - 1) * (w - 1) : h * (w - 1) + (h - 1) * w;
-    } else if (lane == 18) {
-        const int x = v / 100, y = (v / 10) % 10, z = v % 10;
-        ok = x >= 1 && x <= MAXP && y >= 1 && y <= MAXP && z >= 1 && z <= MAXP;
-        c = space == HP3D_H1 ? (x - 1) * (y - 1) * (z - 1)
-                             : x * (y - 1) * (z - 1) + (x - 1) * y * (z - 1) + (x - 1) * (y - 1) * z;
-    }
-    nb = __builtin_amdgcn_readlane(c, 18);
-    const int sum = sf_scan(lane < 18 ? c : 0, [](int x, int y) { return x + y; });
-    ni = __builtin_amdgcn_readlane(sum, 31) + (space == HP3D_H1 ? 8 : 0);
-    return __all(ok);
-}
 
 // Sum over i in [lo, hi) of A[i nb + q0 + q] x[i] for the w <= 64 columns at
 // q0, in lanes q < w: the lanes split into 64 / w groups of w, so that a step

@@ -1419,7 +1419,7 @@ __device__ __forceinline__ void sf_unpack(const double *pk, const SfLay &ly, S *
 // waits in Aii's memory and only the bubble rows are in LDS.
 template <typename T, int NBT, int R, int NW, bool PACKED>
 __device__ __forceinline__ void sf_condense(const ElemArgs &a, const CondArgs &cd, int e, const SfElem &es, double *pk,
-                                            double *kb, const SfLay &ly, double *w, SfSmall<R> &sm, int tid)
+                                            double *kb, const SfLay &ly, double *w, SfSmall<R> &sm, size_t ldc, int tid)
 {
     typedef Mfma<double> MD;
     constexpr int WLD = 16 * NBT + 1;
@@ -1517,7 +1517,7 @@ __device__ __forceinline__ void sf_condense(const ElemArgs &a, const CondArgs &c
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int r = r0 + 4 * j;
-                    acc[j] = aii[r < ni && c <= r ? r + (size_t)c * ni : 0];
+                    acc[j] = aii[r < ni && c <= r ? r + c * ldc : 0];
                 }
             }
             const double *pa = kb + lq * ldb + 16 * tr + lr, *pc = kb + lq * ldb + c;
@@ -1531,8 +1531,8 @@ __device__ __forceinline__ void sf_condense(const ElemArgs &a, const CondArgs &c
                     if (PACKED) {
                         pk[at + j * 4 * r0 + 8 * j * j + 2 * j] = v;
                     } else {
-                        aii[r0 + 4 * j + (size_t)c * ni] = v;
-                        aii[c + (size_t)(r0 + 4 * j) * ni] = v;
+                        aii[r0 + 4 * j + c * ldc] = v;
+                        aii[c + (r0 + 4 * j) * ldc] = v;
                     }
                 }
             } else {
@@ -1545,8 +1545,8 @@ __device__ __forceinline__ void sf_condense(const ElemArgs &a, const CondArgs &c
                         if (PACKED) {
                             pk[at + j * 4 * r0 + 8 * j * j + 2 * j] = v;
                         } else {
-                            aii[r + (size_t)c * ni] = v;
-                            aii[c + (size_t)r * ni] = v;
+                            aii[r + c * ldc] = v;
+                            aii[c + r * ldc] = v;
                         }
                     }
                     if (r == ni && c < ni) bi[c] = bc - up[j];
@@ -1560,7 +1560,7 @@ __device__ __forceinline__ void sf_condense(const ElemArgs &a, const CondArgs &c
         }
         lds_barrier();
     }
-    if (PACKED) sf_unpack(pk, ly, aii, (size_t)ni, ni, wv, NW, lane);
+    if (PACKED) sf_unpack(pk, ly, aii, ldc, ni, wv, NW, lane);
     if (tid == 0 && a.status) a.status[e] = sm.fail ? HP3D_E_FACTOR : (es.negjac ? HP3D_NEG_JACOBIAN : 0);
 }
 
@@ -1673,10 +1673,11 @@ __global__ __launch_bounds__(64 * NW, WPE) void sf_fused_kernel(SingleArgs sa)
                 sf_matrix<SPACE, 6, false>(es, tb, row, pl, js, d, d + dl, POOL - kl - dl, to, 0, 1, tid, WGS);
             else
                 sf_matrix<SPACE, 7, false>(es, tb, row, pl, js, d, d + dl, POOL - kl - dl, to, 0, 1, tid, WGS);
-            sf_condense<T, NBT, R, NW, false>(a, cd, e, es, nullptr, kb, ly, NBT > 1 ? wbuf : pool, sm, tid);
+            sf_condense<T, NBT, R, NW, false>(a, cd, e, es, nullptr, kb, ly, NBT > 1 ? wbuf : pool, sm, n - es.nb, tid);
             continue;
         }
-        sf_condense<T, NBT, R, NW, true>(a, cd, e, es, pool, pool + ly.kb, ly, NBT > 1 ? wbuf : pool + ly.len, sm, tid);
+        sf_condense<T, NBT, R, NW, true>(a, cd, e, es, pool, pool + ly.kb, ly, NBT > 1 ? wbuf : pool + ly.len, sm,
+                                           n - es.nb, tid);
     }
 #endif
 }

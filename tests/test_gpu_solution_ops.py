@@ -66,3 +66,79 @@ def test_gather_and_spmv(gpu, n):
     for got, terms in zip(y.cpu().numpy(), (x[src], vals * x[src])):
         want, mag = np.bincount(row, terms, n), np.bincount(row, np.abs(terms), n)
         assert (np.abs(got - want) <= 1e-12 * mag).all()
+
+
+def codes(space, edge, face, body):
+    """norder of equal edges and faces under a body code, and (n, nb)."""
+    no = np.array([edge] * 12 + [face] * 6 + [body], np.int32)
+    h, v, (x, y, z) = face // 10, face % 10, (int(c) for c in str(body))
+    if space == 0:
+        nb = (x - 1) * (y - 1) * (z - 1)
+        n = 8 + 12 * (edge - 1) + 6 * (h - 1) * (v - 1) + nb
+    else:
+        nb = x * (y - 1) * (z - 1) + (x - 1) * y * (z - 1) + (x - 1) * (y - 1) * z
+        n = 12 * edge + 6 * (h * (v - 1) + (h - 1) * v) + nb
+    return no, n, nb
+
+
+@pytest.mark.parametrize("space,bound,elements", [
+    (0, (64, 16), [(1, 11, 111), (2, 22, 222), (3, 33, 333), (1, 22, 353), (5, 11, 333), (3, 33, 323)]),
+    # interface and bubbles at and beyond what the kernel keeps on the chip (nb = 30 of N = 128)
+    (0, (128, 32), [(4, 44, 444), (1, 46, 643), (1, 46, 422), (2, 44, 543), (5, 34, 111), (4, 44, 333)]),
+    (1, (64, 16), [(1, 11, 111), (2, 22, 222), (4, 11, 122), (4, 11, 222)]),
+    (1, (128, 32), [(2, 33, 222), (3, 22, 322), (1, 33, 332), (2, 33, 321)])])
+@pytest.mark.parametrize("mode", ["packed", "strided", "inplace", "fp32"])
+def test_condense_stored(gpu, space, bound, elements, mode):
+    """stc_batch on random SPD systems with eigenvalues in [1, 5] (N cond eps
+    of the norm is 128 * 5 * 2.2e-16 = 1.4e-13, held to 1e-12); with a leading
+    dimension above N, in place, and K read as FP32."""
+    import torch
+
+    from hp3d_amd import _lib
+
+    lib = _lib.load()
+    rng = np.random.default_rng(sum(bound) + space)
+    el = [codes(space, *x) for x in elements] * 3
+    assert all(n <= bound[0] and nb <= bound[1] for _, n, nb in el)
+    nel, ld = len(el), 0 if mode in ("packed", "fp32") else 131
+    f32 = mode == "fp32"
+    ks, off_k, off_v, off_c, off_s = [], [0], [0], [0], [0]
+    for _, n, nb in el:
+        q = np.linalg.qr(rng.normal(size=(n, n)))[0]
+        k = (q * rng.uniform(1, 5, n)) @ q.T
+        k = 0.5 * (k + k.T)
+        ks.append(k.astype(np.float32).astype(np.float64) if f32 else k)
+        off_k.append(off_k[-1] + (ld or n) * n)
+        off_v.append(off_v[-1] + n)
+        off_c.append(off_c[-1] + (n - nb) ** 2)
+        off_s.append(off_s[-1] + (n - nb) * nb)
+    kin = np.full(off_k[-1], np.nan)
+    for k, o in zip(ks, off_k):
+        kin[o:o + (ld or len(k)) * len(k)].reshape(len(k), -1)[:, :len(k)] = k
+    b = rng.normal(size=off_v[-1])
+    dev = lambda v, t=None: torch.as_tensor(np.asarray(v), dtype=t, device="cuda")
+    kd, bd = dev(kin, torch.float32 if f32 else torch.float64), dev(b)
+    inplace = mode == "inplace"
+    aii = kd if inplace else torch.full((off_c[-1],), float("nan"), dtype=torch.float64, device="cuda")
+    bi = bd if inplace else torch.full_like(bd, float("nan"))
+    xs, xb = (torch.full((m,), float("nan"), dtype=torch.float64, device="cuda") for m in (max(off_s[-1], 1), off_v[-1]))
+    no = dev(np.stack([x[0] for x in el]))
+    offs = [dev(o, torch.int64) for o in (off_k, off_v, off_k if inplace else off_c, off_s)]
+    st = dev(np.arange(nel) % 2, torch.int32)    # every other one with a warning to keep
+    ws = torch.empty(max(lib.hp3d_gpu_stc_workspace(nel, *bound), 1), dtype=torch.uint8, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    rc = lib.hp3d_gpu_stc_batch(space, int(f32), nel, p(no), p(offs[0]), ld, p(kd), p(offs[1]), p(bd), p(offs[2]),
+                                ld if inplace else 0, p(aii), p(bi), p(offs[3]), p(xs), p(xb), p(ws), p(st), *bound, None)
+    torch.cuda.synchronize()
+    assert rc == 0 and np.array_equal(st.cpu().numpy(), np.arange(nel) % 2)
+    aii, bi, xs, xb = (t.cpu().numpy().astype(np.float64) for t in (aii, bi, xs, xb))
+    close = lambda x, y: np.linalg.norm(x - y) <= 1e-12 * max(np.linalg.norm(y), 1.0)
+    for e, (_, n, nb) in enumerate(el):
+        ni, k, be = n - nb, ks[e], b[off_v[e]:off_v[e] + n]
+        x = np.linalg.solve(k[ni:, ni:], np.column_stack([k[ni:, :ni], be[ni:]])) if nb else np.zeros((0, ni + 1))
+        o = off_k[e] if inplace else off_c[e]
+        a = aii[o:o + (ld if inplace else ni) * ni].reshape(ni, -1)[:, :ni]
+        assert close(a, k[:ni, :ni] - k[:ni, ni:] @ x[:, :ni]) and np.array_equal(a, a.T), (e, n, nb)
+        assert close(bi[off_v[e]:off_v[e] + ni], be[:ni] - k[:ni, ni:] @ x[:, ni]), (e, n, nb)
+        assert close(xs[off_s[e]:off_s[e] + ni * nb].reshape(ni, nb), x[:, :ni].T), (e, n, nb)
+        assert close(xb[off_v[e]:off_v[e] + nb], x[:, ni]), (e, n, nb)
