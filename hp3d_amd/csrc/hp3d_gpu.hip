@@ -2583,14 +2583,23 @@ static int launch_single(int space, int precision, const ElemArgs &args, const C
 }
 
 // the sum-factorised element kernel; few elements are split over several
-// workgroups each (their column chunks) until the chip's 256 CUs have three
+// workgroups each (their column chunks) until the chip's 256 CUs have three, 16
+// columns or more to a part (64 H1 p = 4 elements in parts of 16, 32 and 64: 17,
+// 19 and 27 us).  H(curl): up to 64 dofs the pool holds only what the largest
+// point count wants, for three workgroups a CU (8,000 p = 2 elements 0.20 ms,
+// 0.43 with the large pool, 0.41 by the A A^T product); beyond, 8 waves a CU
+// in two workgroups of 4 (FP32 p = 5 1.41 -> 1.10 ms, p = 3 0.27 -> 0.21), 6 in
+// one for the largest FP64 matrices, where fewer columns written at once are
+// the better (512 p = 6 elements 1.25 ms, 1.46 with 8).
 template <typename T>
 static int launch_sf(int space, const ElemArgs &args, int max_ndof, hipStream_t st)
 {
-    const int most = space == HP3D_H1 ? SF_I : 3 * SF_I;
+    const int most = std::min(space == HP3D_H1 ? SF_I : 3 * SF_I, std::max(max_ndof / 16, 1));
     const int parts = std::max(1, std::min(most, 768 / std::max(args.nel, 1)));
     const dim3 grid(args.nel, parts);
     if (space == HP3D_H1) hipLaunchKernelGGL((sf_elem_kernel<T, 0, 256, 5540, 3>), grid, dim3(256), 0, st, args);
+    else if (max_ndof <= BR / 2) hipLaunchKernelGGL((sf_elem_kernel<T, 1, 256, 5660, 3>), grid, dim3(256), 0, st, args);
+    else if (sizeof(T) == 4 || max_ndof <= 2 * BR) hipLaunchKernelGGL((sf_elem_kernel<T, 1, 256, 8674, 2>), grid, dim3(256), 0, st, args);
     else hipLaunchKernelGGL((sf_elem_kernel<T, 1, 384, 8674, 3>), grid, dim3(384), 0, st, args);
     HIPCHK(hipGetLastError());
     return 0;

@@ -1171,7 +1171,7 @@ __global__ __launch_bounds__(WGS, WPE) void sf_elem_kernel(ElemArgs a)
         sf_load<SPACE, WGS>(es, tb, row, pool + (SPACE == 0 ? 6 : 12) * es.nint, [=](int r, double v) { bo[r] = v; }, tid);
     }
     const SfToK<T> to{(T *)a.kout + a.off_k[e], a.ld_k > 0 ? a.ld_k : es.n};
-    const int dl = (sf_fields(SPACE) * es.nint + 1) & ~1;
+    const int dl = (SPACE == 0 ? 6 : 12) * es.nint; // T takes the load fields' place
     auto run = [&](auto mc) __attribute__((always_inline)) {
         sf_matrix<SPACE, decltype(mc)::value, false>(es, tb, row, pl, js, pool, pool + dl, POOL - dl, to, part, nparts,
                                                      tid, WGS);
