@@ -6,14 +6,17 @@
 //   elem_kernel   the BF16 trial for N > 128: one workgroup per (element, 128 x
 //                 128 block of K), A = B^T(geometry) streamed through LDS in
 //                 chunks of quadrature points, K += A A^T on bf16 MFMA.
-//   elem_single_kernel  one workgroup per element with N <= 128: K kept in
-//                 registers over the quadrature, then (nb <= 32) the bubble
-//                 block condensed in the same launch.
+//   sf_fused_kernel  (hp3d_sumfac.h) the same for N <= 128 and nb <= 32 with
+//                 K in LDS, condensed there in the same launch.
+//   elem_single_kernel  the BF16 trial for N <= 128: K kept in registers over
+//                 the quadrature, then (nb <= 32) condensed in the same launch.
+//   stc_small_kernel  condensation of stored matrices with N <= 128 and nb <=
+//                 32, as in sf_fused_kernel.
 //   stc_strip_kernel  one workgroup of 8 waves per element: left-looking
 //                 blocked Cholesky of the bubble block, then [Abi | Bb] in
 //                 register-resident strips through the forward and backward
 //                 sweeps with Aii - Aib X accumulated on the way, FP64 MFMA.
-//   field_kernel  element integrals of finite-element fields (element_error,
+//   field_kernel  (hp3d_sumfac.h) element integrals of finite-element fields (element_error,
 //                 L2 norm and residual, adjoint coefficient gradient).
 //   gather_sum_kernel, csr_spmv_kernel  device assembly and the global operator.
 //   stc_bwd_kernel  xb = BSchur - ASchur xi.
@@ -618,37 +621,6 @@ __device__ inline void write_sym_tile_direct(V acc, int R, int C, int lim, S *ou
     }
 }
 
-// FP32 accumulation with an error-free carry: every ~96 A columns the MFMA
-// accumulator c is folded into a running FP32 sum h by TwoSum
-// (h' = fl(h + c), c' = (h + c) - h' exactly), so c only ever accumulates a
-// few chunks' products on top of a residual and the FP32 rounding of the long
-// k-sum (k = 3Q or 6Q columns) no longer grows with Q.  The tile's value is
-// h + c, used in FP64 by the condensation and rounded once for FP32 output.
-// For FP64 accumulators the carry is absent (Hi is a placeholder).
-template <typename T, typename A> struct Carry {
-    typedef char hi_t;
-    __device__ static inline void zero(hi_t &) {}
-    __device__ static inline void fold(hi_t &, A &) {}
-    __device__ static inline double val(const hi_t &, const A &c, int j) { return (double)c[j]; }
-    __device__ static inline A sum(const hi_t &, const A &c) { return c; }
-};
-template <typename A> struct Carry<float, A> {
-    typedef A hi_t;
-    __device__ static inline void zero(hi_t &h) { h = A{0.f, 0.f, 0.f, 0.f}; }
-    __device__ static inline void fold(hi_t &h, A &c)
-    {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float a = c[j], hh = h[j];
-            float t = hh + a, bp = t - hh;
-            c[j] = (hh - (t - bp)) + (a - bp);
-            h[j] = t;
-        }
-    }
-    __device__ static inline double val(const hi_t &h, const A &c, int j) { return (double)h[j] + (double)c[j]; }
-    __device__ static inline A sum(const hi_t &h, const A &c) { return h + c; }
-};
-
 // bfloat16 operands for the BF16 trial: round to nearest even, 4 values
 // packed per lane as v_mfma_f32_16x16x16_bf16 takes them (lane l supplies
 // A[l % 16][4 (l / 16) + i] and B[4 (l / 16) + i][l % 16], i = 0..3; the
@@ -898,10 +870,10 @@ __global__ __launch_bounds__(WGE, 4) void elem_kernel(ElemArgs a)
     }
 }
 
-// Single-block element kernel (N <= 128): K accumulates in registers over the
-// whole quadrature; then, when the caller asks for it and nb <= NBF, the
-// bubble dofs are condensed in the same launch (the algebra of stc_fwd_herm /
-// stc_fwd_gen, stc.F90:338-509):
+// Single-block element kernel of the BF16 trial (N <= 128): K accumulates in
+// registers over the whole quadrature; then, when the caller asks for it and nb
+// <= NBF, the bubble dofs are condensed in the same launch (the algebra of
+// stc_fwd_herm / stc_fwd_gen, stc.F90:338-509):
 //   Gaussian elimination without pivoting of [Abb | I] (Abb SPD: Abb =
 //   L_u D L_u^T, the pivots D > 0 are the SPD check) gives D and L_u^-1;
 //   then on FP64 MFMA: S = D^-1/2 L_u^-1 [Abi | Bb];  Aii -= S^T S and
@@ -909,20 +881,16 @@ __global__ __launch_bounds__(WGE, 4) void elem_kernel(ElemArgs a)
 //   X = L_u^-T D^-1/2 S = Abb^-1 [Abi | Bb] = [ASchur | BSchur].
 // The A chunks are double buffered: the MFMAs of chunk c are issued before
 // the VALU/LDS work that builds chunk c+1, so the two overlap.
-template <typename T> struct SingleCfg {
-    static constexpr int KCS = sizeof(T) == 4 ? 48 : 24; // A columns per chunk
-};
-
-template <typename T, int SPACE, int R, bool BF = false>
+template <int SPACE, int R>
 __device__ __forceinline__ void single_element(const ElemArgs &a, const CondArgs &cd, const int e,
                                                const int tid)
 {
-    static_assert(!BF || sizeof(T) == 4, "bfloat16 operands accumulate in FP32");
+    typedef float T;
     typedef Mfma<T> M;
     typedef typename M::acc_t acc_t;
     typedef Mfma<double> MD;
     constexpr int NC = SPACE == 0 ? 3 : 6;
-    constexpr int KCS = SingleCfg<T>::KCS;
+    constexpr int KCS = 48;                    // A columns per chunk
     constexpr int QC = KCS / NC;               // points per chunk
     // points per geometry pass (a multiple of QC): 128 for the 128-row H1
     // form, 64 where a third workgroup per CU has to fit in LDS
@@ -940,12 +908,12 @@ __device__ __forceinline__ void single_element(const ElemArgs &a, const CondArgs
     constexpr int LW = NBX + 1;                // leading dimension of L_u^-1
     constexpr int NSLOT = R == BR ? 9 : 3;     // tile slots per wave
     constexpr int UMAX = R == BR ? 5 : 2;      // right-hand-side tiles per wave in the condensation
-    // BF16 trial: the chunk in bfloat16, row-major (a row's KCS values
-    // contiguous, LDB shorts apart), so an MFMA operand (4 consecutive k of
-    // one row) is one 8-byte LDS read
+    // the chunk in bfloat16, row-major (a row's KCS values contiguous, LDB
+    // shorts apart), so an MFMA operand (4 consecutive k of one row) is one
+    // 8-byte LDS read
     constexpr int LDB = KCS + 4;
-    static_assert(!BF || (KCS % 16 == 0 && LDB % 4 == 0), "bf16 chunk layout");
-    constexpr int BUF = BF ? R * LDB / 2 : KCS * LD1; // one A buffer, in T
+    static_assert(KCS % 16 == 0 && LDB % 4 == 0, "bf16 chunk layout");
+    constexpr int BUF = R * LDB / 2;           // one A buffer, in T
     constexpr int AC_D = (2 * BUF * (int)sizeof(T) + 7) / 8;
     constexpr int CW_D = NBX * LDK + NBX * LW + NBX + LD1 + 4 * 16 * 17; // output / condensation workspace
     constexpr int SM_D = AC_D > CW_D ? AC_D : CW_D;
@@ -1032,22 +1000,9 @@ __device__ __forceinline__ void single_element(const ElemArgs &a, const CondArgs
         ti = s < nA ? tiA : tiB;
         tj = s < nA ? tjA + s : tjB + (s - nA);
     };
-    const int offA = tiA * 16 + (lane & 15), offB = tiB * 16 + (lane & 15);
-    int offS[NSLOT];
-#pragma unroll
-    for (int s = 0; s < NSLOT; ++s) {
-        int ti, tj;
-        slot_tile(s, ti, tj);
-        offS[s] = tj * 16 + (lane & 15);
-    }
-    typedef Carry<std::conditional_t<BF, double, T>, acc_t> CY; // no carry under bfloat16 rounding
     acc_t acc[NSLOT];
-    typename CY::hi_t hi[NSLOT];
 #pragma unroll
-    for (int s = 0; s < NSLOT; ++s) {
-        acc[s] = acc_t{0, 0, 0, 0};
-        CY::zero(hi[s]);
-    }
+    for (int s = 0; s < NSLOT; ++s) acc[s] = acc_t{0, 0, 0, 0};
     unsigned valid = 0;
 #pragma unroll
     for (int s = 0; s < NSLOT; ++s) {
@@ -1086,136 +1041,35 @@ __device__ __forceinline__ void single_element(const ElemArgs &a, const CondArgs
             const bool ok = pok && r < n;
             bacc[i] += ok ? bl : 0.0;
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                if constexpr (BF)
-                    reinterpret_cast<short *>(buf)[r * LDB + NC * qt + c] = ok ? f2bf((float)out[c]) : (short)0;
-                else
-                    buf[(NC * qt + c) * LD1 + r] = ok ? (T)out[c] : (T)0;
-            }
+            for (int c = 0; c < NC; ++c)
+                reinterpret_cast<short *>(buf)[r * LDB + NC * qt + c] = ok ? f2bf((float)out[c]) : (short)0;
         }
     };
-    // The slot mask is wave-uniform.  When some of this wave's tiles lie beyond
-    // N (N <= 112), a scalar branch skips their MFMAs; when all are live the
-    // unguarded loop keeps the MFMAs back to back.
+    // The slot mask is wave-uniform: a scalar branch skips the MFMAs of tiles
+    // beyond N.
     const unsigned vmask = __builtin_amdgcn_readfirstlane(valid);
-    const bool all_live = vmask == (1u << NSLOT) - 1;
-    // FP32 H1: the loop specialised per wave, so each slot's operand rows are
-    // compile-time offsets (no per-MFMA select or branch); the FP64 and
-    // H(curl) forms would spill with it.  It runs every slot of the wave also
-    // when some tiles lie beyond N (N <= 112, or 48 in the 64-row form): the
-    // build stores zeros in the rows from N to R, such tiles come out zero,
-    // and no output or condensation step reads a slot outside `valid`
-    constexpr bool SPEC = sizeof(T) == 4 && SPACE == 0 && !BF;
-    // wave W's slots (as set above): rows tiA / tiB, first columns tjA / tjB,
-    // nA slots in row tiA, ns slots in all
-    auto mfma_w = [&](auto wc, const T *buf) {
-        constexpr int W = decltype(wc)::value, P = W & 1;
-        constexpr int TA = R == BR ? W : P, TB = R == BR ? 7 - W : 3 - P;
-        constexpr int JA = R == BR ? W : (W < 2 ? P : P + 3), JB = TB;
-        constexpr int NA = R == BR ? 8 - W : (W < 2 ? 3 : 1 - P), NS = R == BR ? 9 : (W < 2 ? 3 : 2);
-#pragma unroll
-        for (int k0 = 0; k0 < KCS; k0 += 4) {
-            const T *col = buf + (k0 + (lane >> 4)) * LD1 + (lane & 15);
-            const T aA = col[TA * 16], aB = col[TB * 16];
-#pragma unroll
-            for (int s = 0; s < NS; ++s)
-                acc[s] = M::mma(s < NA ? aA : aB, col[(s < NA ? JA + s : JB + (s - NA)) * 16], acc[s]);
-        }
-    };
     const int wv = __builtin_amdgcn_readfirstlane(wave);
-    // The FP32 H1 chunk step with the next chunk's build woven in: after each
-    // k step's MFMAs, one row of the next chunk (rows during the first RPT
-    // k steps), so that the build's VALU and LDS work can issue while the
-    // MFMAs run.  The 128-row form only: the 64-row form's chunk has a third
-    // of the MFMAs to hide the build under, and measured slower with it.
-    auto mfma_build_w = [&](auto wc, const T *buf, int g0, int l0, int gend, T *nbuf) {
-        constexpr int W = decltype(wc)::value, P = W & 1;
-        constexpr int TA = R == BR ? W : P, TB = R == BR ? 7 - W : 3 - P;
-        constexpr int JA = R == BR ? W : (W < 2 ? P : P + 3), JB = TB;
-        constexpr int NA = R == BR ? 8 - W : (W < 2 ? 3 : 1 - P), NS = R == BR ? 9 : (W < 2 ? 3 : 2);
-        constexpr int NKS = KCS / 4;
-        static_assert(RPT <= NKS, "a row per k step");
-        const int lq = l0 + qt;
-        const bool pok = lq < gend;
-        const int lqc = pok ? lq : 0;
-        const unsigned pk = pix[g0 + lqc];
-        const Pt p{(int)(pk & 15), (int)((pk >> 4) & 15), (int)(pk >> 8)};
-        double g[GS];
-#pragma unroll
-        for (int k = 0; k < GS; ++k) g[k] = geo[lqc * GS + k];
-        if (SPLIT) g[9] = g[10] * g[9];
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-            const T *col = buf + (4 * ks + (lane >> 4)) * LD1 + (lane & 15);
-            const T aA = col[TA * 16], aB = col[TB * 16];
-#pragma unroll
-            for (int s = 0; s < NS; ++s)
-                acc[s] = M::mma(s < NA ? aA : aB, col[(s < NA ? JA + s : JB + (s - NA)) * 16], acc[s]);
-            if (ks < RPT) {
-                const int r = rt + TPP * ks;
-                double out[NC];
-                const double bl = a_entries_load<SPACE, true>(dsp[r], p, tv, td, g, out);
-                const bool ok = pok && r < n;
-                bacc[ks] += ok ? bl : 0.0;
-#pragma unroll
-                for (int c = 0; c < NC; ++c) nbuf[(NC * qt + c) * LD1 + r] = ok ? (T)out[c] : (T)0;
-            }
-        }
-    };
     auto mfma = [&](const T *buf) {
-        if constexpr (BF) {
-            // lane l supplies A[l % 16][4 (l / 16) + i] and B[4 (l / 16) + i][l % 16]
-            // (i < 4) of v_mfma_f32_16x16x16_bf16: row l % 16 of a tile, four
-            // consecutive columns of the chunk
-            const short *sb = reinterpret_cast<const short *>(buf) + (lane & 15) * LDB + 4 * (lane >> 4);
+        // lane l supplies A[l % 16][4 (l / 16) + i] and B[4 (l / 16) + i][l % 16]
+        // (i < 4) of v_mfma_f32_16x16x16_bf16: row l % 16 of a tile, four
+        // consecutive columns of the chunk
+        const short *sb = reinterpret_cast<const short *>(buf) + (lane & 15) * LDB + 4 * (lane >> 4);
 #pragma unroll
-            for (int k0 = 0; k0 < KCS; k0 += 16) {
-                const s4_t aA = *reinterpret_cast<const s4_t *>(sb + tiA * 16 * LDB + k0);
-                const s4_t aB = *reinterpret_cast<const s4_t *>(sb + tiB * 16 * LDB + k0);
+        for (int k0 = 0; k0 < KCS; k0 += 16) {
+            const s4_t aA = *reinterpret_cast<const s4_t *>(sb + tiA * 16 * LDB + k0);
+            const s4_t aB = *reinterpret_cast<const s4_t *>(sb + tiB * 16 * LDB + k0);
 #pragma unroll
-                for (int s = 0; s < NSLOT; ++s) {
-                    int ti, tj;
-                    slot_tile(s, ti, tj);
-                    if (vmask & (1u << s))
-                        acc[s] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
-                            s < nA ? aA : aB, *reinterpret_cast<const s4_t *>(sb + tj * 16 * LDB + k0), acc[s], 0, 0,
-                            0);
-                }
-            }
-            return;
-        }
-        if (SPEC) {
-            if constexpr (SPEC) {
-                switch (wv) {
-                case 0: mfma_w(std::integral_constant<int, 0>{}, buf); break;
-                case 1: mfma_w(std::integral_constant<int, 1>{}, buf); break;
-                case 2: mfma_w(std::integral_constant<int, 2>{}, buf); break;
-                default: mfma_w(std::integral_constant<int, 3>{}, buf); break;
-                }
-            }
-        } else if (all_live) {
-#pragma unroll
-            for (int k0 = 0; k0 < KCS; k0 += 4) {
-                const T *col = buf + (k0 + (lane >> 4)) * LD1;
-                const T aA = col[offA], aB = col[offB];
-#pragma unroll
-                for (int s = 0; s < NSLOT; ++s) acc[s] = M::mma(s < nA ? aA : aB, col[offS[s]], acc[s]);
-            }
-        } else {
-#pragma unroll
-            for (int k0 = 0; k0 < KCS; k0 += 4) {
-                const T *col = buf + (k0 + (lane >> 4)) * LD1;
-                const T aA = col[offA], aB = col[offB];
-#pragma unroll
-                for (int s = 0; s < NSLOT; ++s)
-                    if (vmask & (1u << s)) acc[s] = M::mma(s < nA ? aA : aB, col[offS[s]], acc[s]);
+            for (int s = 0; s < NSLOT; ++s) {
+                int ti, tj;
+                slot_tile(s, ti, tj);
+                if (vmask & (1u << s))
+                    acc[s] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                        s < nA ? aA : aB, *reinterpret_cast<const s4_t *>(sb + tj * 16 * LDB + k0), acc[s], 0, 0,
+                        0);
             }
         }
     };
 
-    // fold the FP32 accumulators every 96 columns (2 chunks)
-    constexpr int FOLD_EVERY = KCS >= 48 ? 2 : 4;
-    int nfold = 0;
     for (int g0 = 0; g0 < nint; g0 += GQ) {
         const int gend = min(GQ, nint - g0);
         if (tid < gend) {
@@ -1235,23 +1089,8 @@ __device__ __forceinline__ void single_element(const ElemArgs &a, const CondArgs
         __syncthreads();
         for (int c = 0; c < nch; ++c) {
             T *const cur = ac + (c & 1) * BUF, *const nxt = ac + ((c + 1) & 1) * BUF;
-            if (SPEC && R == BR && c + 1 < nch) {
-                if constexpr (SPEC && R == BR) {
-                    switch (wv) {
-                    case 0: mfma_build_w(std::integral_constant<int, 0>{}, cur, g0, (c + 1) * QC, gend, nxt); break;
-                    case 1: mfma_build_w(std::integral_constant<int, 1>{}, cur, g0, (c + 1) * QC, gend, nxt); break;
-                    case 2: mfma_build_w(std::integral_constant<int, 2>{}, cur, g0, (c + 1) * QC, gend, nxt); break;
-                    default: mfma_build_w(std::integral_constant<int, 3>{}, cur, g0, (c + 1) * QC, gend, nxt); break;
-                    }
-                }
-            } else {
-                mfma(cur);
-                if (c + 1 < nch) build(g0, (c + 1) * QC, gend, nxt);
-            }
-            if ((++nfold & (FOLD_EVERY - 1)) == 0) {
-#pragma unroll
-                for (int s = 0; s < NSLOT; ++s) CY::fold(hi[s], acc[s]);
-            }
+            mfma(cur);
+            if (c + 1 < nch) build(g0, (c + 1) * QC, gend, nxt);
             __syncthreads();
         }
     }
@@ -1265,9 +1104,9 @@ __device__ __forceinline__ void single_element(const ElemArgs &a, const CondArgs
     double *rs = wm + NBX * LW;     // D(j)^-1/2
     double *stg = rs + NBX + LD1;   // 4 x 16 x 17 wave stages
     T *kstage = reinterpret_cast<T *>(stg + wave * (16 * 17));
-    // the FP32 128-row form hands K tiles over through geo[0, NSLOT * 128)
+    // the 128-row form hands K tiles over through geo[0, NSLOT * 128)
     // (as doubles' room); the load vector sits in geo after them
-    constexpr bool KHAND = sizeof(T) == 4 && R == BR;
+    constexpr bool KHAND = R == BR;
     constexpr int BV_OFF = KHAND ? NSLOT * 128 : 0;
     static_assert(GQ * GS >= BV_OFF + R, "load vector beside the K hand-over");
     double *bv = geo + BV_OFF;      // load vector
@@ -1300,7 +1139,7 @@ __device__ __forceinline__ void single_element(const ElemArgs &a, const CondArgs
             if (!(valid & (1u << s))) continue;
             int ti, tj;
             slot_tile(s, ti, tj);
-            write_sym_tile<acc_t, T, M>(CY::sum(hi[s], acc[s]), ti * 16, tj * 16, n, kout, ld, kstage, lane);
+            write_sym_tile<acc_t, T, M>(acc[s], ti * 16, tj * 16, n, kout, ld, kstage, lane);
         }
     };
     if (!cond) {
@@ -1320,7 +1159,7 @@ __device__ __forceinline__ void single_element(const ElemArgs &a, const CondArgs
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             int r = ti * 16 + M::row(lane, j), c = tj * 16 + (lane & 15);
-            double v = CY::val(hi[s], acc[s], j);
+            double v = (double)acc[s][j];
             if (r < n && c < n) {
                 if (c >= ni) kb[(c - ni) * LDK + r] = v;
                 if (r >= ni) kb[(r - ni) * LDK + c] = v;
@@ -1329,8 +1168,7 @@ __device__ __forceinline__ void single_element(const ElemArgs &a, const CondArgs
     }
     // Gaussian elimination of [Abb | I] in the registers of wave EW (L_u^-1
     // and D^-1/2), while the other waves store their tiles of K.  In the
-    // FP32 128-row form EW first hands its own K tiles (the carry folded to
-    // FP32) to the other waves through the geometry buffer, free after the
+    // 128-row form EW first hands its own K tiles to the other waves through the geometry buffer, free after the
     // main loop: its stores would otherwise follow its elimination on the
     // critical path.  Elsewhere EW stores its own afterwards.
     constexpr int EW = 3;
@@ -1341,7 +1179,7 @@ __device__ __forceinline__ void single_element(const ElemArgs &a, const CondArgs
 #pragma unroll
             for (int s = 0; s < NSLOT; ++s) {
                 if (!(valid & (1u << s))) continue;
-                const acc_t v = CY::sum(hi[s], acc[s]);
+                const acc_t v = acc[s];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) khand[s * 256 + 4 * lane + j] = v[j];
             }
@@ -1456,7 +1294,7 @@ __device__ __forceinline__ void single_element(const ElemArgs &a, const CondArgs
         if (R0 >= ni || C0 >= ni) continue;
         d4_t da; // the tile in the accumulator's layout, promoted to FP64
 #pragma unroll
-        for (int j = 0; j < 4; ++j) da[j] = CY::val(hi[s], acc[s], j);
+        for (int j = 0; j < 4; ++j) da[j] = (double)acc[s][j];
         d4_t up = d4_t{0, 0, 0, 0};
         // The FP64 MFMA returns row i of its A operand's rows in register
         // i / 4 of lane group i % 4, the FP32 accumulator holds row
@@ -1511,10 +1349,10 @@ __device__ __forceinline__ void single_element(const ElemArgs &a, const CondArgs
 // one workgroup per element; R = 64 for elements of at most 64 dofs and 16
 // bubbles: half the LDS and a third of the tile registers, so three
 // workgroups share a CU
-template <typename T, int SPACE, int R, bool BF = false>
+template <int SPACE, int R>
 __global__ __launch_bounds__(WG, R == BR ? 2 : 3) void elem_single_kernel(ElemArgs a, CondArgs cd)
 {
-    single_element<T, SPACE, R, BF>(a, cd, blockIdx.x, threadIdx.x);
+    single_element<SPACE, R>(a, cd, blockIdx.x, threadIdx.x);
 }
 
 // ------------------------------------------------------------ condensation
@@ -2522,8 +2360,8 @@ template <int R>
 static int launch_single_bf16(int space, const ElemArgs &args, const CondArgs &cd, hipStream_t st)
 {
     const dim3 grid(args.nel), block(WG);
-    if (space == HP3D_H1) hipLaunchKernelGGL((elem_single_kernel<float, 0, R, true>), grid, block, 0, st, args, cd);
-    else hipLaunchKernelGGL((elem_single_kernel<float, 1, R, true>), grid, block, 0, st, args, cd);
+    if (space == HP3D_H1) hipLaunchKernelGGL((elem_single_kernel<0, R>), grid, block, 0, st, args, cd);
+    else hipLaunchKernelGGL((elem_single_kernel<1, R>), grid, block, 0, st, args, cd);
     HIPCHK(hipGetLastError());
     return 0;
 }
