@@ -156,8 +156,8 @@ class ElementBatch:
     coef (nel,).  Elements are grouped into order bins (the replacement of the
     OpenMP element loop by one launch per bin): bin 0 holds the elements whose
     matrix fits one 128 x 128 block with at most 32 bubbles -- K stays in
-    registers and condensation runs in the same kernel -- and bin 1 the rest
-    (block-tiled element kernel, then the condensation kernel); `rules`
+    LDS and condensation runs in the same kernel -- and bin 1 the rest
+    (element kernel, then the condensation kernel); `rules`
     changes the bin limits and paths (hp3d_amd.tune picks them by timing).
     Internally the elements are stored bin by bin; every accessor takes the
     caller's element index.  Outputs are packed: element i's N_i x N_i matrix starts at
@@ -167,11 +167,11 @@ class ElementBatch:
     FUSED_MAX_NDOF = 128
     FUSED_MAX_NBUBBLE = 32
     # bin rules: an element goes to the first rule whose limits it meets; a
-    # "fused" bin runs the single-block kernel (K in registers, condensation in
-    # the same launch; needs N <= 128, nb <= 32; a bin with N <= 64 and
+    # "fused" bin runs the one-launch kernel (K in LDS, condensation in the
+    # same launch; needs N <= 128, nb <= 32; a bin with N <= 64 and
     # nb <= 16 gets its 64-row form), as a persistent grid when the rule says
-    # "persistent": True; a "two_pass" bin the block-tiled element kernel and
-    # then the blocked condensation
+    # "persistent": True; a "two_pass" bin the element kernel and then the
+    # condensation of stored matrices
     SMALL_MAX_NDOF = 64
     SMALL_MAX_NBUBBLE = 16
     DEFAULT_RULES = ({"max_ndof": 64, "max_nbubble": 16, "path": "fused"},

@@ -3,16 +3,14 @@
 The tunable "tiles" of this path are the two ways an element's stiffness is
 tiled on the chip and the limits that route elements between them:
 
-* the single-block kernel: one workgroup holds the element's whole K
-  (up to 128 x 128) in MFMA accumulator registers, 9 tiles of 16 x 16 per
-  wave, and condenses the bubbles in the same launch; a bin of elements
-  with N <= 64 and nb <= 16 runs its 64-row form (3 tiles per wave, three
+* the fused kernel: one workgroup holds the element's symmetric K (up to
+  128 x 128) in LDS and condenses the bubbles in the same launch; a bin of
+  elements with N <= 64 and nb <= 16 runs its 64-row form (three or four
   workgroups per CU);
-* the block-tiled path: one workgroup per 128 x 128 block of K (or the
-  single-block kernel without condensation for small N), K written to HBM,
-  then the blocked MFMA condensation;
-* for the single-block kernel, one workgroup per element or a persistent
-  grid of 2 workgroups per CU walking the bin's elements.
+* the two-pass path: K written to HBM by the element kernel, then the
+  condensation of stored matrices;
+* for the fused kernel, one workgroup per element or a persistent grid (the
+  workgroups that fit the chip) walking the bin's elements.
 
 For a mesh, ``autotune`` times (HIP events on the launch stream) the full
 element + condensation step of the batch under each candidate rule set --

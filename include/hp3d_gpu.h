@@ -53,13 +53,13 @@ extern "C" {
 #define HP3D_H1 0    /* Poisson: (kappa grad u, grad v) */
 #define HP3D_HCURL 1 /* (mu^-1 curl E, curl F) + (eps E, F), real form */
 
-/* arithmetic of the B^T W B contraction; geometry, Jacobian inverse and the
- * bubble factorisation are always FP64 */
+/* FP64 and FP32 select how K is stored: the arithmetic is FP64 in both, K of
+ * HP3D_FP32 is rounded once, at its store */
 #define HP3D_FP64 0
 #define HP3D_FP32 1
-/* trial: operands rounded to bfloat16, FP32 accumulation (no carry), K stored
- * as FP32; the same kernels as FP32 (single-block and block-tiled), and the
- * condensation as for FP32 */
+/* trial: the B^T W B contraction with operands rounded to bfloat16 and FP32
+ * accumulation, K stored as FP32; geometry, Jacobian inverse and bubble
+ * factorisation in FP64 */
 #define HP3D_BF16 2
 
 /* load selectors (the user getf routine) */
@@ -93,8 +93,8 @@ const char *hp3d_gpu_last_error(void);
 /* Process-wide launch options, read when a batched launch is made (a
  * captured graph keeps the form it was captured with); not synchronised with
  * launches in flight on other threads.  No counterpart in the reference.
- *   HP3D_OPT_PERSISTENT  1: the single-block element kernel runs as a
- *                        persistent grid (2 workgroups per CU walking the
+ *   HP3D_OPT_PERSISTENT  1: the fused kernel runs as a persistent grid (the
+ *                        workgroups that fit the chip, walking the
  *                        elements), 0: one workgroup per element (default) */
 #define HP3D_OPT_PERSISTENT 1
 int hp3d_gpu_set_option(int option, int value);
@@ -143,8 +143,8 @@ int hp3d_gpu_celem(int space, const int norder[19], const int nori_e[12], const 
  *   status[e] (may be NULL): 0, 1 (negative Jacobian) or HP3D_E_ORDER
  * max_ndof bounds N_e over the batch (it sizes the launch grid).
  * workspace: device memory of hp3d_gpu_elem_workspace(space, precision, nel,
- * max_ndof) bytes (the per-element quadrature-point geometry of the
- * block-tiled kernel, N_e > 128); may be NULL when that size is 0.
+ * max_ndof) bytes (used by HP3D_BF16: the per-element quadrature-point
+ * geometry of its kernel for N_e > 128); may be NULL when that size is 0.
  * Replaces the element loop of mumps_sc Step 2 up to elem
  * (mumps_sc.F90:253-259 -> celem_systemI.F90:523).
  */
@@ -154,7 +154,7 @@ int hp3d_gpu_elem_batch(int space, int precision, int nel, const int *norder, co
                         const long long *off_v, double *bout, void *workspace, int *status,
                         int max_ndof, void *stream);
 /* bytes of device workspace hp3d_gpu_elem_batch needs for nel elements of at
- * most max_ndof dofs (0 when the single-block kernel serves the batch).  No
+ * most max_ndof dofs (0 for max_ndof <= 128).  No
  * counterpart in the reference: its elem computes the geometry point by point
  * inside the element loop (elem_opt.F90:101-122). */
 size_t hp3d_gpu_elem_workspace(int space, int precision, int nel, int max_ndof);
@@ -192,7 +192,7 @@ size_t hp3d_gpu_stc_workspace(int nel, int max_ndof, int max_nbubble);
  * celem_systemI.F90:523-534 for nel elements; DEVICE pointers).  Arguments as
  * in hp3d_gpu_elem_batch and hp3d_gpu_stc_batch; max_nbubble bounds nb_e.
  * When max_ndof <= 128 and max_nbubble <= 32 the condensation runs inside the
- * element kernel on the register-resident K (no second pass over HBM); kout
+ * element kernel on K in LDS (no second pass over HBM); kout
  * and bout may then be NULL (K and the full load are not written).  Otherwise
  * K and the load are written and condensed by a second kernel; kout, bout and
  * the hp3d_gpu_celem_workspace(space, precision, nel, max_ndof, max_nbubble)
