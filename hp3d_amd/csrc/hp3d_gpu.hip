@@ -1431,7 +1431,7 @@ __host__ __device__ inline size_t stc_slab(int nbp_max)
     return (size_t)(nbk * (nbk + 1) + 2 * nbk) * 256;
 }
 
-template <typename T, int CW, int MAXR, int NW, int RG, bool RL>
+template <typename T, int CW, int MAXR, int NW, int RG, bool RL, int PF>
 __global__ __launch_bounds__(64 * NW) void stc_strip_kernel(StcArgs a)
 {
     typedef Mfma<double> MD;
@@ -1923,22 +1923,27 @@ __global__ __launch_bounds__(64 * NW) void stc_strip_kernel(StcArgs a)
             for (int g = 0; g < RG; ++g)
 #pragma unroll
                 for (int t = 0; t < CT; ++t) accA[g][t] = d4_t{0.0, 0.0, 0.0, 0.0};
-            // Aib(ri, kb) = K(ri, ni + kb), the values of step p + 1 loaded
-            // during step p
-            T nA[RG][4];
-            auto ld_A = [&](int p) {
+            // Aib(ri, kb) = K(ri, ni + kb), the values of step p + PF loaded
+            // during step p (they come from HBM)
+            T nA[PF][RG][4];
+            auto ld_A = [&](int u, int p) {
 #pragma unroll
                 for (int g = 0; g < RG; ++g) {
                     const int ri = 16 * (I0 + NW * g) + lr;
 #pragma unroll
                     for (int s2 = 0; s2 < 4; ++s2) {
                         const int kb = 16 * p + 4 * s2 + lq;
-                        nA[g][s2] = K[(ri < ni && kb < nb) ? (size_t)ri + (size_t)(ni + kb) * ldk : 0];
+                        nA[u][g][s2] = K[(ri < ni && kb < nb) ? (size_t)ri + (size_t)(ni + kb) * ldk : 0];
                     }
                 }
             };
-            ld_A(0);
-            for (int p = 0; p < nbk; ++p) {
+#pragma unroll
+            for (int u = 0; u < PF; ++u) ld_A(u, min(u, nbk - 1));
+            for (int p0 = 0; p0 < nbk; p0 += PF)
+#pragma unroll
+            for (int u = 0; u < PF; ++u) { // (a body for each of the PF sets of registers)
+                const int p = p0 + u;
+                if (p >= nbk) break;
                 double cA[RG][4];
 #pragma unroll
                 for (int g = 0; g < RG; ++g) {
@@ -1946,10 +1951,10 @@ __global__ __launch_bounds__(64 * NW) void stc_strip_kernel(StcArgs a)
 #pragma unroll
                     for (int s2 = 0; s2 < 4; ++s2) {
                         const int kb = 16 * p + 4 * s2 + lq;
-                        cA[g][s2] = (ri < ni && kb < nb) ? (double)nA[g][s2] : 0.0;
+                        cA[g][s2] = (ri < ni && kb < nb) ? (double)nA[u][g][s2] : 0.0;
                     }
                 }
-                ld_A(min(p + 1, nbk - 1));
+                ld_A(u, min(p + PF, nbk - 1));
 #pragma unroll
                 for (int s2 = 0; s2 < 4; ++s2) {
 #pragma unroll
@@ -2107,14 +2112,21 @@ static void launch_stc(StcArgs a, int max_nbubble, hipStream_t st)
     }
     // 64-column strips (2 block rows per wave) up to 256 bubbles, with the
     // register-resident Cholesky up to 240; 32-column strips (4 block rows
-    // per wave) beyond
+    // per wave) beyond.  Last argument: how many steps ahead Aib is loaded for
+    // Aib X.  Three steps hide the most of HBM's latency (1,728 H(curl) p = 5
+    // elements with their matrices 7.44 -> 6.91 ms, two 7.31, four spill: 7.42);
+    // up to four block rows there are not enough steps (2,744 p = 3 elements
+    // one 1.148 ms, two 1.137, three 1.19); the 32-column form has no registers
+    // to spare (343 p = 6 elements 10.26 ms, two 10.9, three 10.2)
     const int nbp = rnd16(max_nbubble);
-    if (nbp <= 240)
-        hipLaunchKernelGGL((stc_strip_kernel<T, 64, 2, 8, 2, true>), dim3(a.nel), dim3(512), 0, st, a);
+    if (nbp <= 64)
+        hipLaunchKernelGGL((stc_strip_kernel<T, 64, 2, 8, 2, true, 2>), dim3(a.nel), dim3(512), 0, st, a);
+    else if (nbp <= 240)
+        hipLaunchKernelGGL((stc_strip_kernel<T, 64, 2, 8, 2, true, 3>), dim3(a.nel), dim3(512), 0, st, a);
     else if (nbp <= 256)
-        hipLaunchKernelGGL((stc_strip_kernel<T, 64, 2, 8, 2, false>), dim3(a.nel), dim3(512), 0, st, a);
+        hipLaunchKernelGGL((stc_strip_kernel<T, 64, 2, 8, 2, false, 3>), dim3(a.nel), dim3(512), 0, st, a);
     else
-        hipLaunchKernelGGL((stc_strip_kernel<T, 32, 4, 8, 2, false>), dim3(a.nel), dim3(512), 0, st, a);
+        hipLaunchKernelGGL((stc_strip_kernel<T, 32, 4, 8, 2, false, 1>), dim3(a.nel), dim3(512), 0, st, a);
 }
 
 struct BwdArgs {
