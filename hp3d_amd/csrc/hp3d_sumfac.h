@@ -159,7 +159,7 @@ __device__ __forceinline__ int sf_scan(int x, F f)
 template <int SPACE, int WGS>
 __device__ __forceinline__ bool sf_setup(const ElemArgs &a, int e, SfElem &es, double *xg, int tid, SfFused fu = {0, 0, 0, 0, 0, 0})
 {
-        const int nx = a.ngeo <= XS_MAX ? 3 * a.ngeo : 0;
+    const int nx = a.ngeo <= XS_MAX ? 3 * a.ngeo : 0;
     constexpr int NX = WGS > 3 * XS_MAX ? 1 : 2;
     static_assert(NX * WGS > 3 * XS_MAX, "staged values");
     double xv[NX];
@@ -362,7 +362,8 @@ __device__ __forceinline__ double sf_map(const SfElem &es, const SfTab &tb, cons
 }
 
 // Metric fields and load of every quadrature point, q = (qA mB + qB) mC + qC,
-// field f at d[f * nint + q], the weights folded in (elem_opt.F90:101-122).  Returns true when a point of this thread has det < 0.
+// field f at d[f * nint + q], the weights folded in (elem_opt.F90:101-122).
+// Returns true when a point of this thread has det < 0.
 // The load and the metric of a point are evaluated by different waves, side by
 // side (the lower half of the workgroup has the metric).
 template <int SPACE, bool STAGED>
@@ -1139,9 +1140,9 @@ __device__ __forceinline__ void sf_load(const SfElem &es, const SfTab &tb, const
 // an element share its column chunks, so that a few elements fill the chip.
 // Bound by writing K (9.6 GB for 4,096 H(curl) p = 5 elements in FP64, at the
 // rate of a large copy 2 ms): the element + condensation step of that mesh
-// took 54.3 ms with the A A^T product on MFMA tiles (41 ms of it the product)
-// and takes 17.1 ms; element matrices of 990 H(curl) p = 4 elements in FP32
-// 1.53 -> 0.38 ms.
+// took 54.4 ms with the A A^T product on MFMA tiles (41 ms of it the product)
+// and takes 15.7 ms (3.7 ms of it this kernel); element matrices of 990
+// H(curl) p = 4 elements in FP32 1.53 -> 0.24 ms.
 template <typename T, int SPACE, int WGS, int POOL, int WPE>
 __global__ __launch_bounds__(WGS, WPE) void sf_elem_kernel(ElemArgs a)
 {
