@@ -38,6 +38,7 @@
 
 #include "../../include/hp3d_gpu.h"
 #include "hp3d_tables.h"
+#include "hp3d_sumfac_layout.h"
 
 typedef double d4_t __attribute__((ext_vector_type(4)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
@@ -189,7 +190,6 @@ struct ElemArgs {
 // block-tiled path: MAXQ points, then the negative-Jacobian flag
 __host__ __device__ constexpr int geo_stride(int space) { return space == 0 ? 10 : 21; }
 __host__ __device__ constexpr size_t geo_slab(int space) { return (size_t)MAXQ * geo_stride(space) + 2; }
-constexpr int XS_MAX = 27; // geometry nodes staged in LDS by the geometry code
 
 __device__ inline void getf(int load, const double *x, double *f)
 {
@@ -2393,31 +2393,24 @@ static int fused_grid(int nel, int per_cu, dim3 &grid)
 }
 
 // The fused kernel: 64 rows and 16 bubbles when the batch's bounds allow it.
-// The pools are the smallest that hold every element in one of the modes, the
-// waves those that fill a CU with the workgroups that the pools let in
-// (workgroups x waves, 13,824 H1 p = 3 elements in FP64): 3 x 4 0.46 ms, 4 x 4
-// at 128 registers 0.46, 4 x 3 at 168 registers 0.45, 4 x 2 0.49, 4 x 1 0.56.
-// 8,000 H1 p = 4 elements: 2 x 8 at 128 registers 0.78 ms in FP64 and 0.68 in
-// FP32, 2 x 4 at 256 0.78 and 0.73; 6 waves at 168 registers leave a CU one
-// workgroup (a SIMD would have to take four of their waves): 1.1.
-// 8,000 H(curl) p = 2 elements: 3 x 4 0.30 ms, 2 x 4 0.42.
+template <typename T, int SHAPE> static int launch_fused_shape(const SingleArgs &sa, hipStream_t st)
+{
+    constexpr SfShape s = sf_shape(SHAPE);
+    dim3 grid;
+    if (int r = fused_grid(sa.a.nel, s.per_cu, grid)) return r;
+    hipLaunchKernelGGL((sf_fused_kernel<T, s.space, s.rows, s.nbt, s.waves, s.pool, s.wpe>), grid, dim3(64 * s.waves), 0,
+                       st, sa);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
 template <typename T>
 static int launch_fused(int space, const ElemArgs &args, const CondArgs &cd, int max_ndof, int max_nbubble,
                         hipStream_t st)
 {
     const bool small = max_ndof <= BR / 2 && max_nbubble <= NBF / 2;
-    dim3 grid;
     const SingleArgs sa{args, cd};
-    if (int r = fused_grid(args.nel, space == HP3D_H1 ? (small ? 4 : 2) : (small ? 3 : 1), grid)) return r;
-    if (space == HP3D_H1) {
-        if (small) hipLaunchKernelGGL((sf_fused_kernel<T, 0, 64, 1, 3, 4500, 3>), grid, dim3(192), 0, st, sa);
-        else hipLaunchKernelGGL((sf_fused_kernel<T, 0, 128, 2, 8, 8352, 4>), grid, dim3(512), 0, st, sa);
-    } else {
-        if (small) hipLaunchKernelGGL((sf_fused_kernel<T, 1, 64, 1, 4, 5660, 3>), grid, dim3(256), 0, st, sa);
-        else hipLaunchKernelGGL((sf_fused_kernel<T, 1, 128, 2, 8, 13932, 2>), grid, dim3(512), 0, st, sa);
-    }
-    HIPCHK(hipGetLastError());
-    return 0;
+    if (space == HP3D_H1) return small ? launch_fused_shape<T, SF_H1_64>(sa, st) : launch_fused_shape<T, SF_H1_128>(sa, st);
+    return small ? launch_fused_shape<T, SF_HCURL_64>(sa, st) : launch_fused_shape<T, SF_HCURL_128>(sa, st);
 }
 
 // the single-launch path of a batch whose elements have at most max_ndof

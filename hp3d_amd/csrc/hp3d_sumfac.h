@@ -24,18 +24,7 @@
 
 __constant__ SfTables c_sf = make_sf_tables();
 
-constexpr int SF_I = MAXP + 1;                   // 1D functions per direction
-__host__ __device__ constexpr int sf_comps(int space) { return space == 0 ? 1 : 3; }
-// fields per point: metric (6 symmetric entries; H(curl) curl, then mass) and load
-__host__ __device__ constexpr int sf_fields(int space) { return space == 0 ? 7 : 15; }
-__host__ __device__ constexpr int sf_ttabs(int space) { return space == 0 ? 8 : 9; }
 __host__ __device__ constexpr int sf_sym(int r, int s) { return r <= s ? r * (5 - r) / 2 + s : s * (5 - s) / 2 + r; }
-
-// doubles of the staged geometry nodes, the coefficient and the node map
-constexpr int SF_XG = 3 * XS_MAX + 1 + (SF_I * SF_I * SF_I + 3) / 4;
-
-// How the block of K is kept while its entries are computed (sf_choose)
-enum { SF_STREAM = 0, SF_DIRECT = 1, SF_HOLD = 2 };
 
 // One element.  m[] and everything indexed like it goes by role: 0 = B, 1 = A,
 // 2 = C, with dir[role] the element direction of the role and rol[] its
@@ -48,91 +37,18 @@ struct SfElem {
     int n, nb, nh, m[3], dir[3], rol[3], nint, ok, negjac, np, mode;
 };
 
-// where a pool of doubles holds one element's packed K (PK), fields and T:
-// which roles the directions take, and whether K's entries go straight to LDS
-// (SF_DIRECT: packed K, fields and at least one row of T fit together), stay in
-// registers until T is done with (SF_HOLD: all of T fits, one pencil pair per
-// thread at MC = 5, two at MC = 4), or are recomputed (SF_STREAM)
-struct SfFused {
-    int pool, wgs, nbx; // nbx: the most bubbles it condenses
-    int xg;               // pool doubles taken by the staged nodes
-    int h5, h4;           // pencil pairs a thread holds at MC = 5 and 4 (0: never)
-};
-
-// Storage of one element's symmetric K in LDS: rows r < ni as a packed lower
-// triangle, entry (r, c) at r (r + 1) / 2 + c, then the bubble rows at an odd
-// stride, whole up to their diagonal, and zero rows up to a multiple of four
-// (an element that is not condensed has all rows packed: ni = n)
-struct SfLay {
-    int ni, kb, ldb, len;
-    __host__ __device__ SfLay(int n, int nb, int nbx)
-    {
-        ni = nb <= nbx ? n - nb : n;
-        kb = ni * (ni + 1) / 2;
-        ldb = n | 1;
-        len = (kb + ((n - ni + 3) & ~3) * ldb + 1) & ~1;
-    }
-    __device__ __forceinline__ int row(int r) const
-    {
-        const int t = __mul24(r, r + 1) >> 1, b = kb + __mul24(r - ni, ldb);
-        return r < ni ? t : b;
-    }
-};
-
-// Roles of the directions and the mode of one element (orders md[], n dofs).
-// The streaming kernel takes (B, A, C) = (x, y, z), so that consecutive lanes
-// run along consecutive bubble rows.  A fused kernel takes the C that costs the
-// fewest steps, counting whole passes of the workgroup over the pencil pairs,
-// of those that fit its pool.
+// roles of the directions and the mode of one element (orders md[], n dofs)
 template <int SPACE>
 __device__ __forceinline__ void sf_choose(SfElem &es, const int (&md)[3], int n, SfFused fu)
 {
-    int best = SF_STREAM, cC = 2, cA = 1, cost = 0x7fffffff;
-    if (fu.pool > 0) {
-        const int Q = md[0] * md[1] * md[2], pk = SfLay(n, es.nb, fu.nbx).len;
-        const int dl = sf_fields(SPACE) * Q + fu.xg, dk = (SPACE == 0 ? 6 : 12) * Q; // with and without the load
-        if (md[0] == md[1] && md[1] == md[2]) { // nothing to choose but the mode
-            const int m = md[0], one = sf_ttabs(SPACE) * m * ((m + 1) & ~1), P = m * m;
-            if (pk + max(dl, dk + one) <= fu.pool) best = SF_DIRECT;
-            else if (max(dl, dk + m * (m + 1) / 2 * one) <= fu.pool && P * (P + 1) / 2 <= (m == 5 ? fu.h5 : m == 4 ? fu.h4 : 0) * fu.wgs)
-                best = SF_HOLD;
-        } else {
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            const int C = 2 - i, x = C == 0 ? 1 : 0, y = C == 2 ? 1 : 2; // the other two, x < y
-            const int mC = md[C], mcp = (mC + 1) & ~1, mx = md[x], my = md[y], lo = min(mx, my), hi = max(mx, my);
-            const int P = (SPACE == 0 ? 1 : 3) * mx * my, items = P * (P + 1) / 2;
-            auto price = [&](int mB) __attribute__((always_inline)) {
-                return ((items + fu.wgs - 1) / fu.wgs) * (9 * mB * mC + 2 * mC * mC * mC + 4 * mC * mC);
-            };
-            // direct: B the shorter of the two (its sums are the inner loop)
-            const bool direct = pk + max(dl, dk + sf_ttabs(SPACE) * lo * mcp) <= fu.pool;
-            const int cap = mC == 5 ? fu.h5 * fu.wgs : mC == 4 ? fu.h4 * fu.wgs : 0;
-            const bool hold = items <= cap && max(dl, dk + 4 * lo * (lo + 1) * hi * mcp) <= fu.pool;
-            const int mode = direct ? SF_DIRECT : hold ? SF_HOLD : SF_STREAM;
-            const int c = direct ? price(lo) : hold ? price(hi) : 0x7fffffff;
-            if (mode != SF_STREAM && c < cost) {
-                cost = c;
-                best = mode;
-                cC = C;
-                cA = (mode == SF_DIRECT) == (my >= mx) ? y : x;
-                if (mx == my) cA = y;
-            }
-        }
-        }
-        if (best == SF_STREAM) { // the longest direction for C
-            cC = md[2] >= md[0] && md[2] >= md[1] ? 2 : md[1] >= md[0] ? 1 : 0;
-            cA = cC == 1 ? 2 : 1;
-        }
-    }
-    const int cB = 3 - cC - cA;
-    es.mode = best;
-    es.dir[0] = cB;
-    es.dir[1] = cA;
-    es.dir[2] = cC;
+    const SfRoles ro = sf_roles<SPACE>(md, n, es.nb, fu);
+    es.mode = ro.mode;
+    es.dir[0] = ro.b;
+    es.dir[1] = ro.a;
+    es.dir[2] = ro.c;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        const int r = d == cB ? 0 : d == cA ? 1 : 2;
+        const int r = d == ro.b ? 0 : d == ro.a ? 1 : 2;
         es.rol[d] = r;
         es.m[r] = md[d];
     }
@@ -1587,9 +1503,10 @@ __global__ __launch_bounds__(64 * NW, WPE) void sf_fused_kernel(SingleArgs sa)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int WGS = 64 * NW;
-    constexpr int H5 = SPACE == 0 && R == BR ? (325 + WGS - 1) / WGS : 0, H4 = H5 ? (666 + WGS - 1) / WGS : 0;
-    // (the pool of the 128-row H(curl) form holds every element's K, fields and T)
-    constexpr bool HOLD = H5 > 0, STREAM = SPACE == 0 || R < BR;
+    constexpr SfShape SH{SPACE, R, NBT, NW, POOL, WPE, 0};
+    constexpr SfFused FU = sf_limits(SH);
+    constexpr int H5 = FU.h5, H4 = FU.h4;
+    constexpr bool HOLD = H5 > 0, STREAM = sf_streams(SH);
     __shared__ SfElem es;
     __shared__ SfTab tb;
     __shared__ SfSmall<R> sm;
@@ -1616,7 +1533,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void sf_fused_kernel(SingleArgs sa)
         __asm__ volatile("" : "+v"(tid));
         double *const xg = NBT > 1 ? wbuf : pool + POOL - SF_XG;
         unsigned short *const gmap = reinterpret_cast<unsigned short *>(xg + 3 * XS_MAX + 1);
-        const bool ok = sf_setup<SPACE, WGS>(a, e, es, xg, tid, SfFused{POOL, WGS, 16 * NBT, NBT > 1 ? 0 : SF_XG, H5, H4});
+        const bool ok = sf_setup<SPACE, WGS>(a, e, es, xg, tid, FU);
         if (!ok || es.n > a.max_ndof || es.n > R) { // invalid codes, or above the caller's bound
             if (tid == 0 && a.status) a.status[e] = ok ? HP3D_E_ARG : HP3D_E_ORDER;
             continue;
@@ -1670,7 +1587,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void sf_fused_kernel(SingleArgs sa)
                                   es.nb <= 16 * NBT ? cd.aii + cd.off_c[e] : nullptr, n - es.nb, ly.ldb};
             // (with the pools of the launches, elements whose longest
             // direction has fewer functions never come here)
-            if (HOLD && es.m[2] == 6)
+            if (HOLD && sf_stream_mc(SH, es.m[2]) == 6)
                 sf_matrix<SPACE, 6, false>(es, tb, row, pl, js, d, d + dl, POOL - kl - dl, to, 0, 1, tid, WGS);
             else
                 sf_matrix<SPACE, 7, false>(es, tb, row, pl, js, d, d + dl, POOL - kl - dl, to, 0, 1, tid, WGS);
