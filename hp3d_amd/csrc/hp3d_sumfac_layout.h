@@ -27,6 +27,9 @@ constexpr int SF_XG = 3 * XS_MAX + 1 + (SF_I * SF_I * SF_I + 3) / 4;
 // ms in FP64 and 0.68 in FP32, 2 x 4 at 256 0.78 and 0.73; 6 waves at 168
 // registers leave a CU one workgroup (a SIMD would have to take four of their
 // waves): 1.1.  8,000 H(curl) p = 2 elements: 3 x 4 0.30 ms, 2 x 4 0.42.
+// The 64-row H(curl) pool is the smallest in which every element with at most
+// six functions a direction is direct (N = 64, nb = 9: 5,728), so that the one
+// streamed template is of seven.
 struct SfShape {
     int space, rows, nbt, waves, pool, wpe, per_cu;
 };
@@ -35,7 +38,7 @@ HP3D_HD constexpr SfShape sf_shape(int i)
 {
     return i == SF_H1_64    ? SfShape{0, 64, 1, 3, 4500, 3, 4}
          : i == SF_H1_128   ? SfShape{0, 128, 2, 8, 8352, 4, 2}
-         : i == SF_HCURL_64 ? SfShape{1, 64, 1, 4, 5660, 3, 3}
+         : i == SF_HCURL_64 ? SfShape{1, 64, 1, 4, 5728, 3, 3}
                             : SfShape{1, 128, 2, 8, 13932, 2, 1};
 }
 

@@ -65,3 +65,19 @@ def test_edges_above_the_interior_h1(gpu, most):
     pick = np.array([e for e in ok if packed(int(n[e]), int(nb[e])) > 8352][:12])
     assert pick.size >= 4
     condensed_at_the_end(0, no[pick], oe[pick], of[pick], sum(most))
+
+
+@pytest.mark.parametrize("interior,edges,faces,size", [(221, [5] * 12, [21] * 3 + [11] * 3, (64, 1)),
+                                                       (122, [5] * 12, [12] * 3 + [11] * 3, (64, 1)),
+                                                       (441, [4] * 5 + [5] * 7, [11] * 6, (64, 9)),
+                                                       (144, [4] * 5 + [5] * 7, [11] * 6, (64, 9)),
+                                                       (111, [5] * 12, [11] * 3 + [21] * 3, (63, 0)),
+                                                       (111, [6] + [5] * 7 + [6] + [5] * 3, [11] * 6, (62, 0))])
+def test_six_functions_a_direction_hcurl(gpu, interior, edges, faces, size):
+    """64 rows in H(curl): K and the fields of 6 x 6 x 6 points just fit (and
+    those of 7 x 6 x 7, the last, do not)."""
+    no = np.array([edges + faces + [interior]] * 3, np.int32)
+    assert (np.array(ndof(1, no[0])) == size).all()
+    rng = np.random.default_rng(interior)
+    oe = rng.integers(0, 2, (3, 12)).astype(np.int32)
+    condensed_at_the_end(1, no, oe, rng.integers(0, 8, (3, 6)).astype(np.int32), interior)
