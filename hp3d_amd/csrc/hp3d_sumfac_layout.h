@@ -29,7 +29,8 @@ constexpr int SF_XG = 3 * XS_MAX + 1 + (SF_I * SF_I * SF_I + 3) / 4;
 // waves): 1.1.  8,000 H(curl) p = 2 elements: 3 x 4 0.30 ms, 2 x 4 0.42.
 // The 64-row H(curl) pool is the smallest in which every element with at most
 // six functions a direction is direct (N = 64, nb = 9: 5,728), so that the one
-// streamed template is of seven.
+// streamed template is of seven; the 128-row one the smallest in which every
+// element is direct (N = 128, nb = 29 at 7 x 7 x 7 points: 14,223).
 struct SfShape {
     int space, rows, nbt, waves, pool, wpe, per_cu;
 };
@@ -39,7 +40,7 @@ HP3D_HD constexpr SfShape sf_shape(int i)
     return i == SF_H1_64    ? SfShape{0, 64, 1, 3, 4500, 3, 4}
          : i == SF_H1_128   ? SfShape{0, 128, 2, 8, 8352, 4, 2}
          : i == SF_HCURL_64 ? SfShape{1, 64, 1, 4, 5728, 3, 3}
-                            : SfShape{1, 128, 2, 8, 13932, 2, 1};
+                            : SfShape{1, 128, 2, 8, 14224, 2, 1};
 }
 
 // How the block of K is kept while its entries are computed (sf_roles)

@@ -81,3 +81,16 @@ def test_six_functions_a_direction_hcurl(gpu, interior, edges, faces, size):
     rng = np.random.default_rng(interior)
     oe = rng.integers(0, 2, (3, 12)).astype(np.int32)
     condensed_at_the_end(1, no, oe, rng.integers(0, 8, (3, 6)).astype(np.int32), interior)
+
+
+@pytest.mark.parametrize("interior,faces,size", [(252, [33, 33, 23, 22, 11, 11], (128, 21)), (616, [33, 11, 23, 11, 33, 11], (128, 25)),
+                                                 (226, [11, 13, 33, 33, 22, 11], (128, 26)), (234, [33, 33, 14, 11, 11, 11], (128, 29)),
+                                                 (432, [11, 12, 11, 33, 33, 11], (126, 29)), (225, [33, 33, 23, 11, 11, 11], (124, 21))])
+def test_seven_functions_a_direction_hcurl(gpu, interior, faces, size):
+    """128 rows in H(curl), edges of order 6: K and the fields of 7 x 7 x 7
+    points come to the pool's end."""
+    no = np.array([[6] * 12 + faces + [interior]] * 3, np.int32)
+    assert (np.array(ndof(1, no[0])) == size).all()
+    rng = np.random.default_rng(interior)
+    oe = rng.integers(0, 2, (3, 12)).astype(np.int32)
+    condensed_at_the_end(1, no, oe, rng.integers(0, 8, (3, 6)).astype(np.int32), interior)

@@ -106,7 +106,7 @@ def program(tmp_path_factory):
     return str(exe)
 
 
-@pytest.mark.parametrize("shape", [0, 1, 2], ids=["h1_64", "h1_128", "hcurl_64"])
+@pytest.mark.parametrize("shape", [0, 1, 2, 3], ids=["h1_64", "h1_128", "hcurl_64", "hcurl_128"])
 def test_every_element_fits(program, shape):
     r = subprocess.run([program, str(shape)], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
