@@ -2020,8 +2020,9 @@ __global__ __launch_bounds__(64 * NW) void stc_strip_kernel(StcArgs a)
 // (128 rows) or five (64 rows) workgroups a CU.  Bound by reading K's triangle
 // and writing Aii; the strips below, which go through a workspace, are built
 // for blocks of more than one MFMA tile column: 4,080 H1 p = 4 elements 1.07 ->
-// 0.23 ms.  An element whose triangle does not fit (N near 128 with 28 bubbles
-// or more) keeps only its bubble rows in LDS.
+// 0.23 ms.  An element whose packed K is larger than the pool (SfLay's len: N =
+// 124..128 with some numbers of bubbles) keeps only its bubble rows in LDS; one
+// without bubbles is copied.
 template <typename T, int R, int NBT, int NW, int POOL, int WPE>
 __global__ __launch_bounds__(64 * NW, WPE) void stc_small_kernel(StcArgs sa)
 {
@@ -2057,6 +2058,15 @@ __global__ __launch_bounds__(64 * NW, WPE) void stc_small_kernel(StcArgs sa)
     const size_t ldk = sa.ld_k > 0 ? (size_t)sa.ld_k : (size_t)n, ldc = sa.ld_c > 0 ? (size_t)sa.ld_c : (size_t)ni;
     const double *b = sa.bin + sa.off_v[e];
     double *const aii = sa.aii + sa.off_c[e];
+    if (nb == 0) { // nothing to condense: copied as it is, also unsymmetric (stc.F90:207)
+        for (int k = tid; k < n * n; k += WGS) {
+            const int c = k / n, r = k - c * n;
+            aii[r + c * ldc] = (double)K[r + c * ldk];
+        }
+        for (int k = tid; k < n; k += WGS) (sa.bi + sa.off_v[e])[k] = b[k];
+        if (tid == 0 && sa.status && sa.status[e] != HP3D_NEG_JACOBIAN) sa.status[e] = 0;
+        return;
+    }
     const SfLay ly(n, nb, 16 * NBT);
     const bool packed = ly.len <= POOL;
     // column c of K's upper triangle is row c of SfLay's; without room for all

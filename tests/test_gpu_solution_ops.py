@@ -142,3 +142,49 @@ def test_condense_stored(gpu, space, bound, elements, mode):
         assert close(bi[off_v[e]:off_v[e] + ni], be[:ni] - k[:ni, ni:] @ x[:, ni]), (e, n, nb)
         assert close(xs[off_s[e]:off_s[e] + ni * nb].reshape(ni, nb), x[:, :ni].T), (e, n, nb)
         assert close(xb[off_v[e]:off_v[e] + nb], x[:, ni]), (e, n, nb)
+
+
+@pytest.mark.parametrize("space,bound,elements", [(0, (64, 16), [(1, 11, 111), (5, 11, 111), (2, 22, 231)]),
+                                                  (0, (128, 32), [(1, 11, 111), (6, 33, 111), (5, 44, 166)]),
+                                                  (1, (64, 16), [(1, 11, 111), (4, 12, 121), (5, 11, 161)]),
+                                                  (1, (128, 32), [(1, 11, 111), (6, 11, 116), (4, 23, 111)])])
+@pytest.mark.parametrize("mode", ["packed", "strided", "inplace", "fp32"])
+def test_condense_without_bubbles(gpu, space, bound, elements, mode):
+    """An element without bubbles comes through as it is, to the bit, also an
+    unsymmetric one, among elements of a batch with other bounds."""
+    import torch
+
+    from hp3d_amd import _lib
+
+    lib = _lib.load()
+    rng = np.random.default_rng(sum(bound) + space + 1)
+    el = [codes(space, *x) for x in elements] * 3
+    assert all(n <= bound[0] and nb == 0 for _, n, nb in el)
+    nel, ld = len(el), 0 if mode in ("packed", "fp32") else 131
+    f32, inplace = mode == "fp32", mode == "inplace"
+    off_k = np.concatenate([[0], np.cumsum([(ld or n) * n for _, n, _ in el])])
+    off_v = np.concatenate([[0], np.cumsum([n for _, n, _ in el])])
+    off_c = np.concatenate([[0], np.cumsum([n * n for _, n, _ in el])])
+    dt = torch.float32 if f32 else torch.float64
+    dev = lambda v, t=None: torch.as_tensor(np.asarray(v), dtype=t, device="cuda")
+    kd, bd = dev(rng.normal(size=off_k[-1]), dt), dev(rng.normal(size=off_v[-1]))
+    kin, b = kd.cpu().numpy().astype(np.float64), bd.cpu().numpy()
+    aii = kd if inplace else torch.full((int(off_c[-1]),), float("nan"), dtype=torch.float64, device="cuda")
+    bi = bd if inplace else torch.full_like(bd, float("nan"))
+    none = torch.zeros(1, dtype=torch.float64, device="cuda")
+    no = dev(np.stack([x[0] for x in el]))
+    offs = [dev(o, torch.int64) for o in (off_k, off_v, off_k if inplace else off_c, [0] * nel)]
+    st = dev(np.arange(nel) % 3, torch.int32)    # a warning to keep, and a stale code
+    ws = torch.empty(lib.hp3d_gpu_stc_workspace(nel, *bound), dtype=torch.uint8, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    rc = lib.hp3d_gpu_stc_batch(space, int(f32), nel, p(no), p(offs[0]), ld, p(kd), p(offs[1]), p(bd), p(offs[2]),
+                                ld if inplace else 0, p(aii), p(bi), p(offs[3]), p(none), p(none), p(ws), p(st), *bound, None)
+    torch.cuda.synchronize()
+    assert rc == 0 and np.array_equal(st.cpu().numpy(), np.arange(nel) % 3 == 1)
+    aii, bi = aii.cpu().numpy(), bi.cpu().numpy()
+    assert np.array_equal(bi, b)
+    for e, (_, n, _) in enumerate(el):
+        k = kin[off_k[e]:off_k[e] + (ld or n) * n].reshape(n, -1)[:, :n]
+        o = off_k[e] if inplace else off_c[e]
+        a = aii[o:o + (ld if inplace else n) * n].reshape(n, -1)[:, :n]
+        assert np.array_equal(a, k), (e, n)
