@@ -1966,7 +1966,11 @@ __global__ __launch_bounds__(64 * NW) void stc_strip_kernel(StcArgs a)
                     }
                 }
             }
-            // Aii = Kii - Aib X (both triangles), Bi = Bi - Aib BSchur
+            // Aii = Kii - Aib X (both triangles), Bi = Bi - Aib BSchur.  A wave reads
+            // only entries of Kii that it writes itself, so that in place no
+            // other wave's Aii is taken for Kii: above the strip's diagonal
+            // block those of the mirrored tile (lanes along a column), in it
+            // the tile's own
 #pragma unroll
             for (int g = 0; g < RG; ++g) {
                 const int I = I0 + NW * g;
@@ -1978,7 +1982,9 @@ __global__ __launch_bounds__(64 * NW) void stc_strip_kernel(StcArgs a)
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         const int r = 16 * I + MD::row(lane, j), c = c0 + 16 * t + lr;
-                        kraw[j] = K[(r < ni && c < ni) ? (size_t)c + (size_t)r * ldk : 0];
+                        const bool own = 16 * I >= c0;
+                        const int a0 = own ? r : c, a1 = own ? c : r;
+                        kraw[j] = K[(r < ni && c < ni) ? (size_t)a0 + (size_t)a1 * ldk : 0];
                     }
                     // mirrored entries (c, r) first, straight from the
                     // accumulator: lanes run along c, i.e. along the rows of column r

@@ -188,3 +188,51 @@ def test_condense_without_bubbles(gpu, space, bound, elements, mode):
         o = off_k[e] if inplace else off_c[e]
         a = aii[o:o + (ld if inplace else n) * n].reshape(n, -1)[:, :n]
         assert np.array_equal(a, k), (e, n)
+
+
+@pytest.mark.parametrize("space,edge,body", [(0, 2, 455), (0, 5, 555), (0, 6, 666), (1, 3, 333), (1, 4, 444), (1, 6, 555), (1, 6, 666)])
+def test_condense_in_place_by_strips(gpu, space, edge, body):
+    """Systems of more than 32 bubbles condensed in place, as stc_fwd does on
+    ALOC: the same bits as out of place, and within N cond eps (882 * 5 *
+    2.2e-16 = 9.8e-13, held to 1e-11) of numpy."""
+    import torch
+
+    from hp3d_amd import _lib
+
+    lib = _lib.load()
+    rng = np.random.default_rng(edge + body)
+    no, n, nb = codes(space, edge, 11 * edge, body)
+    assert nb > 32
+    nel, ld, ni = 6, n + 5, n - nb
+    q = np.linalg.qr(rng.normal(size=(n, n)))[0]
+    ks = [(q * rng.uniform(1, 5, n)) @ q.T for _ in range(nel)]
+    kin = np.full((nel, n, ld), np.nan)
+    for e, k in enumerate(ks):
+        kin[e, :, :n] = 0.5 * (k + k.T)
+    b = rng.normal(size=(nel, n))
+    dev = lambda v, t=None: torch.as_tensor(np.ascontiguousarray(v), dtype=t, device="cuda")
+    nod, off_k, off_v, off_s = (dev(v, t) for v, t in ((np.stack([no] * nel), torch.int32), (np.arange(nel) * n * ld, torch.int64),
+                                                       (np.arange(nel) * n, torch.int64), (np.arange(nel) * nb * ni, torch.int64)))
+    ws = torch.empty(lib.hp3d_gpu_stc_workspace(nel, n, nb), dtype=torch.uint8, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    out = []
+    for inplace in (False, True):
+        kd, bd = dev(kin.reshape(-1)), dev(b.reshape(-1))
+        aii, bi = (kd, bd) if inplace else (torch.full_like(kd, float("nan")), torch.full_like(bd, float("nan")))
+        xs = torch.full((nel * nb * ni,), float("nan"), dtype=torch.float64, device="cuda")
+        xb = torch.full_like(bd, float("nan"))
+        st = torch.zeros(nel, dtype=torch.int32, device="cuda")
+        rc = lib.hp3d_gpu_stc_batch(space, 0, nel, p(nod), p(off_k), ld, p(kd), p(off_v), p(bd), p(off_k), ld, p(aii),
+                                    p(bi), p(off_s), p(xs), p(xb), p(ws), p(st), n, nb, None)
+        torch.cuda.synchronize()
+        assert rc == 0 and (st == 0).all()
+        out.append([aii.view(nel, n, ld)[:, :ni, :ni].cpu().numpy(), bi.view(nel, n)[:, :ni].cpu().numpy(),
+                    xs.view(nel, ni, nb).cpu().numpy(), xb.view(nel, n)[:, :nb].cpu().numpy()])
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
+    close = lambda x, y: np.linalg.norm(x - y) <= 1e-11 * max(np.linalg.norm(y), 1.0)
+    for e in range(nel):
+        k, (aii, bi, xs, xb) = kin[e, :, :n], [v[e] for v in out[1]]
+        x = np.linalg.solve(k[ni:, ni:], np.column_stack([k[ni:, :ni], b[e, ni:]]))
+        assert close(aii, k[:ni, :ni] - k[:ni, ni:] @ x[:, :ni]) and close(bi, b[e, :ni] - k[:ni, ni:] @ x[:, ni]), e
+        assert close(xs, x[:, :ni].T) and close(xb, x[:, ni]), e
