@@ -2288,29 +2288,39 @@ __global__ __launch_bounds__(GATHER_WG) void gather_sum_kernel(long long nout, c
     out[t] = s;
 }
 
-// y = A x for a CSR matrix (FP64 values, int32 column indices): 16 lanes per
+// y = A x for a CSR matrix (FP64 values, int32 column indices): LPR lanes per
 // row, each lane striding over the row's nonzeros, four of them in flight, then
 // a shuffle reduction.  HBM bound: 12 bytes per nonzero plus the gathered x
 // (29.4M nonzeros 0.101 -> 0.089 ms, 4.0 TB/s; 26.8M in rows of 190 0.083 ->
 // 0.067; 32 lanes with four in flight 0.096, 64 lanes 0.122).  The global
-// condensed systems have tens to hundreds of nonzeros per row.
-constexpr int SPMV_LPR = 16;
+// condensed systems have tens to hundreds of nonzeros per row; rows of at most
+// LPR take one product a lane instead of four loads of which three are not used
+// (100,000 rows of 8: 9.9 -> 5.9 us).  Few rows take 32 lanes, for more waves
+// (10,000 rows of 400: 18.8 us, 21.2 with 16; 81: 4.5 and 5.0), which beyond
+// has no more to give (20,000 rows of 400: 38.0 and 37.9; of 190: 19.4 and 19.0).
+constexpr long long SPMV_FEW = 16384;
+template <int LPR>
 __global__ __launch_bounds__(WG) void csr_spmv_kernel(long long nrows, const long long *indptr,
                                                      const int *indices, const double *vals,
                                                      const double *x, double *y)
 {
     constexpr int U = 4;
-    const long long row = (long long)blockIdx.x * (WG / SPMV_LPR) + threadIdx.x / SPMV_LPR;
-    const int sub = threadIdx.x % SPMV_LPR;
+    const long long row = (long long)blockIdx.x * (WG / LPR) + threadIdx.x / LPR;
+    const int sub = threadIdx.x % LPR;
     double s = 0.0;
     if (row < nrows) {
         const long long end = indptr[row + 1];
-        for (long long j0 = indptr[row] + sub; j0 < end; j0 += U * SPMV_LPR) {
+        long long j0 = indptr[row] + sub;
+        if (__all(end - j0 + sub <= LPR)) {
+            if (j0 < end) s = vals[j0] * x[indices[j0]];
+            j0 = end;
+        }
+        for (; j0 < end; j0 += U * LPR) {
             double v[U], xv[U];
             int c[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const long long j = min(j0 + u * SPMV_LPR, end - 1);
+                const long long j = min(j0 + u * LPR, end - 1);
                 v[u] = vals[j];
                 c[u] = indices[j];
             }
@@ -2318,10 +2328,10 @@ __global__ __launch_bounds__(WG) void csr_spmv_kernel(long long nrows, const lon
             for (int u = 0; u < U; ++u) xv[u] = x[c[u]];
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                if (j0 + u * SPMV_LPR < end) s += v[u] * xv[u];
+                if (j0 + u * LPR < end) s += v[u] * xv[u];
         }
     }
-    for (int off = SPMV_LPR / 2; off > 0; off >>= 1) s += __shfl_down(s, off, SPMV_LPR);
+    for (int off = LPR / 2; off > 0; off >>= 1) s += __shfl_down(s, off, LPR);
     if (row < nrows && sub == 0) y[row] = s;
 }
 
@@ -2962,10 +2972,12 @@ int hp3d_gpu_csr_spmv(long long nrows, const long long *indptr, const int *indic
     if (nrows < 0) return HP3D_E_ARG;
     if (nrows == 0) return 0;
     if (!indptr || !indices || !vals || !x || !y) return HP3D_E_ARG;
-    long long nblk = (nrows + WG / SPMV_LPR - 1) / (WG / SPMV_LPR);
+    const int lpr = nrows < SPMV_FEW ? 32 : 16;
+    const long long nblk = (nrows + WG / lpr - 1) / (WG / lpr);
     if (nblk > 0x7fffffffLL) return HP3D_E_ARG;
-    hipLaunchKernelGGL(csr_spmv_kernel, dim3((unsigned)nblk), dim3(WG), 0, (hipStream_t)stream,
-                       nrows, indptr, indices, vals, x, y);
+    const dim3 grid((unsigned)nblk), block(WG);
+    if (lpr == 32) hipLaunchKernelGGL(csr_spmv_kernel<32>, grid, block, 0, (hipStream_t)stream, nrows, indptr, indices, vals, x, y);
+    else hipLaunchKernelGGL(csr_spmv_kernel<16>, grid, block, 0, (hipStream_t)stream, nrows, indptr, indices, vals, x, y);
     HIPCHK(hipGetLastError());
     return 0;
 }

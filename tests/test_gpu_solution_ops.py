@@ -68,6 +68,32 @@ def test_gather_and_spmv(gpu, n):
         assert (np.abs(got - want) <= 1e-12 * mag).all()
 
 
+@pytest.mark.parametrize("n", [3, 16383, 16384])
+@pytest.mark.parametrize("longest", [1, 16, 17, 32, 33, 130])
+def test_spmv_row_lengths(gpu, n, longest):
+    """Rows of up to one product a lane and beyond, few rows and many, empty
+    ones among them."""
+    import torch
+
+    from hp3d_amd import _lib
+
+    lib = _lib.load()
+    rng = np.random.default_rng(n + longest)
+    cnt = rng.integers(0, longest + 1, n)
+    cnt[:: 7] = longest
+    ptr = np.concatenate([[0], np.cumsum(cnt)])
+    src = rng.integers(0, n, ptr[-1])
+    vals, x = rng.normal(size=ptr[-1]), rng.normal(size=n)
+    t = [torch.as_tensor(v, device="cuda") for v in (ptr, src.astype(np.int32), vals, x)]
+    y = torch.full((n,), float("nan"), dtype=torch.float64, device="cuda")
+    p = lambda v: ctypes.c_void_p(v.data_ptr())
+    assert lib.hp3d_gpu_csr_spmv(n, *(p(v) for v in t), p(y), None) == 0
+    torch.cuda.synchronize()
+    row, terms = np.repeat(np.arange(n), cnt), vals * x[src]
+    want, mag = np.bincount(row, terms, n), np.bincount(row, np.abs(terms), n)
+    assert (np.abs(y.cpu().numpy() - want) <= 1e-12 * mag).all()
+
+
 def codes(space, edge, face, body):
     """norder of equal edges and faces under a body code, and (n, nb)."""
     no = np.array([edge] * 12 + [face] * 6 + [body], np.int32)
