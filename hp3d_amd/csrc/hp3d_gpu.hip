@@ -2130,17 +2130,21 @@ static void launch_stc(StcArgs a, int max_nbubble, hipStream_t st)
     // register-resident Cholesky up to 240; 32-column strips (4 block rows
     // per wave) beyond.  Last argument: how many steps ahead Aib is loaded for
     // Aib X.  Three steps hide the most of HBM's latency (1,728 H(curl) p = 5
-    // elements with their matrices 7.44 -> 6.91 ms, two 7.31, four spill: 7.42);
-    // up to four block rows there are not enough steps (2,744 p = 3 elements
-    // one 1.148 ms, two 1.137, three 1.19); the 32-column form has no registers
-    // to spare (343 p = 6 elements 10.26 ms, two 10.9, three 10.2)
+    // elements 5.79 ms with one, 5.26 with three, which spill 72 bytes a lane;
+    // four spill more and were slower than two); up to four block rows there
+    // are not enough steps (2,744 p = 3 elements one and two 0.92 ms, three
+    // more); the 32-column form has no registers to spare.  FP32 matrices, half
+    // the bytes, have less to hide: p = 5 5.00 ms with one step, 5.06 with two,
+    // 5.16 with three; up to four block rows H1 p = 5 0.956 with one, 0.945
+    // with two.
+    constexpr int PF = sizeof(T) == 8 ? 3 : 1;
     const int nbp = rnd16(max_nbubble);
     if (nbp <= 64)
         hipLaunchKernelGGL((stc_strip_kernel<T, 64, 2, 8, 2, true, 2>), dim3(a.nel), dim3(512), 0, st, a);
     else if (nbp <= 240)
-        hipLaunchKernelGGL((stc_strip_kernel<T, 64, 2, 8, 2, true, 3>), dim3(a.nel), dim3(512), 0, st, a);
+        hipLaunchKernelGGL((stc_strip_kernel<T, 64, 2, 8, 2, true, PF>), dim3(a.nel), dim3(512), 0, st, a);
     else if (nbp <= 256)
-        hipLaunchKernelGGL((stc_strip_kernel<T, 64, 2, 8, 2, false, 3>), dim3(a.nel), dim3(512), 0, st, a);
+        hipLaunchKernelGGL((stc_strip_kernel<T, 64, 2, 8, 2, false, PF>), dim3(a.nel), dim3(512), 0, st, a);
     else
         hipLaunchKernelGGL((stc_strip_kernel<T, 32, 4, 8, 2, false, 1>), dim3(a.nel), dim3(512), 0, st, a);
 }
