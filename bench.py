@@ -14,11 +14,14 @@ forms      the same for the batched FP64 form and for the plain FP64 drop-in
            (one C-ABI call per element from the host, as the reference's
            OpenMP loop would make it, from one thread and from a pool of
            host threads)
-roofline   the step's launches: the reference's flops (k N (N+1) per element,
-           its DSYRK, plus the condensation count) over their mean duration
-           (HIP events on the launch stream); the kernels do fewer (sum
-           factorisation), so the fraction is a rate of the reference's work
-           and may pass 1
+roofline   the step's launches: the bytes they cannot do without (inputs once,
+           outputs once) over their mean duration (HIP events on the launch
+           stream) against the HBM peak, the nearest roof of the
+           sum-factorised kernels (they stay below it on the length of an
+           element's chain of phases; traffic is what they do move);
+           reference_* is the same time priced in the reference's flops
+           (k N (N+1) per element, its DSYRK, plus the condensation count), of
+           which the kernels do only a part
 cpu_baseline  the oracle's OpenMP element loop in the reference's own form
            (DSYRK, DGETRF/DGETRS/DGEMM from the host OpenBLAS) on a bounded
            sample of the same mesh, on this host's cores
@@ -39,7 +42,7 @@ sys.path.insert(0, ROOT)
 
 METRIC = ("element matrices/s + condensed DOF/s: plain FP64 vs batched FP32 at "
           "≤1e-6 rel err")
-PEAK = {"fp64": 78.6e12, "fp32": 157.3e12, "hbm": 8.0e12}
+PEAK = {"hbm": 8.0e12}
 
 WORKLOADS = {
     "cfg1": "Poisson H1, 32x32x32 hexahedra on the unit cube, uniform p=4 (125 dofs, 125 Gauss "
@@ -290,6 +293,14 @@ def kernel_names(batch):
     return " ; ".join(parts)
 
 
+def step_bytes(batch, k_bytes):
+    """Bytes of one step: codes, geometry, coefficients and offsets in; K, load,
+    Aii, Bi, ASchur, BSchur and status out."""
+    n, ni, nb = (np.asarray(v, np.float64) for v in (batch._n, batch._ni, batch._nb))
+    head = 37 * 4 + 24 * batch.ngeo + 8 + 4 * 8 + 4
+    return float((head + k_bytes * n * n + 8 * (n + ni * ni + ni + nb * ni + nb)).sum())
+
+
 def traffic_of(workload):
     """HBM bytes per step from the committed counter summary of this workload
     (FETCH_SIZE and WRITE_SIZE passes, scaled by a plain copy's reading)."""
@@ -390,7 +401,7 @@ def measure(workload, args, headline):
         forms["bf16_trial"] = {"element_matrices_per_s": nel / s16, "ms_per_step": s16 * 1e3,
                                "k_err_max": k16max, "k_err_median": k16med, "aii_err_max": a16max,
                                "note": "bfloat16 operands, FP32 accumulation, the FP32 form's bins"}
-    achieved = (fk + fc) / (e32 * 1e-3)
+    achieved = {k: step_bytes(batch, 4 if k == "fp32" else 8) / (ms * 1e-3) for k, ms in (("fp32", e32), ("fp64", e64))}
     entry = {
         "workload": "%s: %s" % (workload, WORKLOADS[workload]),
         "elements": nel,
@@ -402,12 +413,16 @@ def measure(workload, args, headline):
         "forms": forms,
         "fp32_vs_fp64_error": {"k_max": kmax, "k_median": kmed, "aii_max": amax,
                                "aii_median": amed},
-        "roofline": {"bound": "mfma", "achieved": achieved / 1e12, "peak": PEAK["fp32"] / 1e12,
-                     "unit": "TFLOP/s", "frac": achieved / PEAK["fp32"],
+        "roofline": {"bound": "hbm", "achieved": achieved["fp32"] / 1e9, "peak": PEAK["hbm"] / 1e9,
+                     "unit": "GB/s", "frac": achieved["fp32"] / PEAK["hbm"],
                      "traffic": traffic_of(workload), "kernel": kernel_names(batch),
-                     "flops_per_launch": fk + fc, "flops_k": fk, "flops_condensation": fc},
-        "roofline_fp64": {"achieved": (fk + fc) / (e64 * 1e-3) / 1e12, "peak": PEAK["fp64"] / 1e12,
-                          "unit": "TFLOP/s", "frac": (fk + fc) / (e64 * 1e-3) / PEAK["fp64"]},
+                     "bytes_per_launch": step_bytes(batch, 4),
+                     "reference_flops_per_launch": fk + fc, "reference_flops_k": fk,
+                     "reference_flops_condensation": fc,
+                     "reference_tflop_per_s": (fk + fc) / (e32 * 1e-3) / 1e12},
+        "roofline_fp64": {"bound": "hbm", "achieved": achieved["fp64"] / 1e9, "peak": PEAK["hbm"] / 1e9,
+                          "unit": "GB/s", "frac": achieved["fp64"] / PEAK["hbm"],
+                          "reference_tflop_per_s": (fk + fc) / (e64 * 1e-3) / 1e12},
         "tuning": tuning,
     }
     if workload == "cfg2":

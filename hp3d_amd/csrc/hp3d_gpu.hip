@@ -2504,7 +2504,7 @@ static int launch_elem(int space, int precision, const ElemArgs &args, int max_n
 // ------------------------------------------------ allocation-free scratch
 
 // Device scratch of hp3d_gpu_celem_batch_noalloc: the workspace of its two-pass
-// bins (per-element geometry slabs, then the condensation slabs), one copy per
+// bins (the element pass's, which BF16 alone reads, then the condensation slabs), one copy per
 // device, held from module load until the process ends.  In host code the
 // array's name is only a stand-in: kernels get the address that
 // hipGetSymbolAddress returns for the current device (scratch_dev).
@@ -2705,7 +2705,9 @@ int hp3d_gpu_elem_batch(int space, int precision, int nel, const int *norder, co
 size_t hp3d_gpu_elem_workspace(int space, int precision, int nel, int max_ndof)
 {
     if (nel <= 0 || max_ndof <= 0 || (space != HP3D_H1 && space != HP3D_HCURL)) return 0;
-    if (max_ndof <= BR) return 0; // single-block kernel
+    // one size for every precision: callers size a workspace once and pass it
+    // with another (only the BF16 kernel for N > 128 reads it)
+    if (max_ndof <= BR) return 0;
     return (size_t)nel * geo_slab(space) * sizeof(double);
 }
 
@@ -2718,7 +2720,8 @@ size_t hp3d_gpu_stc_workspace(int nel, int max_ndof, int max_nbubble)
 size_t hp3d_gpu_celem_workspace(int space, int precision, int nel, int max_ndof, int max_nbubble)
 {
     if (max_ndof <= BR && max_nbubble <= NBF) return 0; // fused
-    // the geometry pass and the condensation use the same memory one after the other
+    // the element pass (BF16: its geometry) and the condensation use the same
+    // memory one after the other
     return std::max(hp3d_gpu_elem_workspace(space, precision, nel, max_ndof),
                     hp3d_gpu_stc_workspace(nel, max_ndof, max_nbubble));
 }

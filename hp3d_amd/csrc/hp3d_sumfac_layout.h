@@ -21,16 +21,21 @@ constexpr int SF_XG = 3 * XS_MAX + 1 + (SF_I * SF_I * SF_I + 3) / 4;
 // One launch shape: elements of at most `rows` dofs and 16 nbt bubbles, `waves`
 // waves with a pool of `pool` doubles, wpe waves per SIMD (launch bound), per_cu
 // workgroups on a CU.  The waves are those that fill a CU with the workgroups
-// that the pools let in (workgroups x waves, 13,824 H1 p = 3 elements in FP64):
-// 3 x 4 0.46 ms, 4 x 4 at 128 registers 0.46, 4 x 3 at 168 registers 0.45,
-// 4 x 2 0.49, 4 x 1 0.56.  8,000 H1 p = 4 elements: 2 x 8 at 128 registers 0.78
-// ms in FP64 and 0.68 in FP32, 2 x 4 at 256 0.78 and 0.73; 6 waves at 168
-// registers leave a CU one workgroup (a SIMD would have to take four of their
-// waves): 1.1.  8,000 H(curl) p = 2 elements: 3 x 4 0.30 ms, 2 x 4 0.42.
+// that the pools let in.  Measured (workgroups x waves of a CU):
+//   13,824 H1 p = 3 elements, FP64, and p = 2: 4 x 3 at 168 registers 0.386 and
+//   0.228 ms; 4 x 4 at 128 0.385 and 0.246; 3 x 4 0.438 and 0.280; 4 x 2 0.417
+//   and 0.228; 4 x 1 0.484 and 0.244;
+//   8,000 H1 p = 4 elements, FP64 and FP32: 2 x 8 at 128 registers 0.612 and
+//   0.612 ms; 2 x 4 at 256 0.662 and 0.650; 6 waves at 168 registers leave a CU
+//   one workgroup (a SIMD would have to take four of their waves): 1.03 and 1.06;
+//   8,000 H(curl) p = 2 elements: 3 x 4 0.281 ms, 3 x 3 0.305, 3 x 2 0.320, 2 x 4
+//   (a pool of 8,000) 0.338.
 // The 64-row H(curl) pool is the smallest in which every element with at most
 // six functions a direction is direct (N = 64, nb = 9: 5,728), so that the one
 // streamed template is of seven; the 128-row one the smallest in which every
-// element is direct (N = 128, nb = 29 at 7 x 7 x 7 points: 14,223).
+// element is direct (N = 128, nb = 29 at 7 x 7 x 7 points: 14,223).  The 128-row
+// H1 pool is about what two workgroups leave of a CU's LDS: the packed K of a
+// whole p = 4 element; what is larger is streamed.
 struct SfShape {
     int space, rows, nbt, waves, pool, wpe, per_cu;
 };

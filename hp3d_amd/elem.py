@@ -254,8 +254,8 @@ class ElementBatch:
         self.workspace = torch.empty(self._workspace_bytes(FP32) // 8 + 1, dtype=torch.float64, device=dev)
 
     def _workspace_bytes(self, precision):
-        """Workspace of the per-bin calls: the geometry of the block-tiled
-        element pass and the condensation slabs (one after the other)."""
+        """Workspace of the per-bin calls: the element pass's (read by BF16
+        alone) and the condensation slabs, one after the other."""
         lib = _lib.load()
         ws = 8
         for _, cnt, mnd, mnb in self.bins:

@@ -143,8 +143,9 @@ int hp3d_gpu_celem(int space, const int norder[19], const int nori_e[12], const 
  *   status[e] (may be NULL): 0, 1 (negative Jacobian) or HP3D_E_ORDER
  * max_ndof bounds N_e over the batch (it sizes the launch grid).
  * workspace: device memory of hp3d_gpu_elem_workspace(space, precision, nel,
- * max_ndof) bytes (used by HP3D_BF16: the per-element quadrature-point
- * geometry of its kernel for N_e > 128); may be NULL when that size is 0.
+ * max_ndof) bytes (asked for in every precision, used by HP3D_BF16 alone: the
+ * per-element quadrature-point geometry of its kernel for N_e > 128); may be
+ * NULL when that size is 0.
  * Replaces the element loop of mumps_sc Step 2 up to elem
  * (mumps_sc.F90:253-259 -> celem_systemI.F90:523).
  */
@@ -163,6 +164,8 @@ size_t hp3d_gpu_elem_workspace(int space, int precision, int nel, int max_ndof);
  * Static condensation of nel element systems already in device memory
  * (stc_fwd_wrapper + stc_fwd_herm, stc.F90:182-416), FP64 arithmetic:
  *   kin  at off_k[e], ld_k (0 = N_e), FP64 or FP32 by `precision`
+ *        (symmetric: either triangle may be the one read; an element without
+ *        bubbles is copied as it is)
  *   bin  at off_v[e]
  *   aii  at off_c[e], ld_c (0 = ni_e): condensed matrix (may alias kin when
  *        precision is FP64, off_c == off_k and ld_c == ld_k: in place as ALOC)
@@ -171,7 +174,8 @@ size_t hp3d_gpu_elem_workspace(int space, int precision, int nel, int max_ndof);
  *   workspace: device memory of hp3d_gpu_stc_workspace(nel, max_ndof,
  *   max_nbubble) bytes (one slab per element: the bubble block's Cholesky
  *   factor in 16 x 16 tiles, its transformed copy and the inverted diagonal
- *   blocks; independent of max_ndof)
+ *   blocks; independent of max_ndof); asked for at every size, used when
+ *   max_ndof > 128 or max_nbubble > 32
  *   max_ndof, max_nbubble bound N_e and nb_e over the batch (an element above
  *   them reports HP3D_E_ARG in status[e])
  *   status[e]: 0, a negative code, or 1 when status[e] already held 1 (the
